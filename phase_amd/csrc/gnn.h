@@ -47,13 +47,14 @@ struct GnnState {
   DBuf<float> resC, resQ, resDq, resG;  // residual objective: out / sd, A c, dloss/dq, A dloss/dq
   DBuf<__bf16> h;      // (L+1) x n x 64
   DBuf<__bf16> agg, pre;  // L x n x 64
-  DBuf<__bf16> pre0, dpre;
-  DBuf<float> dh, dSA;    // n x 64, n x 128
+  DBuf<__bf16> pre0;
+  DBuf<float> dh, dagg;   // n x 64, two of n x 64 (the layer above's and this one's)
+  DBuf<float> ahat;       // graph weights, SELL layout
+  DBuf<double> stage;     // operands of the host entry points, 3 n
   DBuf<float> gmean;      // L x 64
-  DBuf<float> cvec;       // L x 64 (b + g Wg)
+  DBuf<float> cvec;       // L x 64 (b + g Wg); backward: gterm in the first 64
   DBuf<float> partials;
   DBuf<double> scal;      // [0] rms scale s, [1] loss
-  DBuf<unsigned> counter;
   // captured (residual, correction) pairs, solver order, FP32
   int captureEvery = 0, maxPairs = 0, nPairs = 0;
   std::vector<int> pendingSnap;           // pair slots of the running solve

@@ -40,40 +40,43 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int H = kGnnH;
-constexpr int kRowsPerWave = 16;
-constexpr int kWgRows = 64;     // rows per workgroup in row-parallel kernels
-constexpr int kChunkRows = 2048;  // rows per workgroup in weight-gradient kernels
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+
+// Rows of a layer kernel's tile (16 per wavefront): one SELL-64 slice, so a
+// tile's row offsets are a single pair of scalars.
+constexpr int kTileRows = 64;
+// Workgroups of the layer kernels.  Each takes a contiguous run of tiles (its
+// weights stay in LDS and its sums in registers over the run), and every
+// workgroup leaves one partial record: more of them cost the finishing sums,
+// fewer leave the gathers with too few wavefronts in flight (a forward
+// workgroup holds 18 KB of LDS, a backward one 46 KB: three per CU).  Twice as
+// many of either: mean 10.0 us instead of 7.2, backward layer 91 us instead of
+// 79 (200,000 rows).
+constexpr int kFwdGroups = 1280;
+constexpr int kBwdGroups = 768;
+constexpr int kFinThreads = 1024;  // 64 columns x 16 slices of the partial records
+
+struct Tiles {
+  int n, per, groups;  // tiles, tiles per workgroup, workgroups
+};
+Tiles tilesFor(int n, int groups) {
+  Tiles t;
+  t.n = std::max(1, (n + kTileRows - 1) / kTileRows);
+  t.per = (t.n + groups - 1) / groups;
+  t.groups = (t.n + t.per - 1) / t.per;
+  return t;
+}
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
-
-// Graph weight of SELL entry idx of solver row `row`: a_ij / (sd_i sd_j), or
-// 0 for the diagonal and padding.
-template <class T>
-__device__ __forceinline__ float ahat(const int *__restrict__ col, const T *__restrict__ val,
-                                      const float *__restrict__ sd, int idx, int row, int &c) {
-  c = col[idx];
-  if (c < 0 || c == row) return 0.f;
-  return (float)val[idx] / (sd[row] * sd[c]);
-}
-
 int gridFor1(long n) { return (int)std::max<long>(1, std::min<long>((n + kRedBlock - 1) / kRedBlock, 1024)); }
 
 // ---------------------------------------------------------------- features
-__global__ void kGnnScale(int n, const float *__restrict__ valDiag, const float *__restrict__ rowsumIn,
-                          float *__restrict__ sd, float *__restrict__ rowsum) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    sd[i] = sqrtf(fabsf(valDiag[i]));
-    rowsum[i] = rowsumIn[i];
-  }
-}
-
-// diag and row-sum ratio from the SELL FP32 copy of A
+// sd_i = sqrt|a_ii| and the row-sum ratio from the SELL FP32 copy of A
 __global__ void kGnnDiag(int n, const int *__restrict__ sliceOff, const int *__restrict__ col,
-                         const float *__restrict__ val, float *__restrict__ diag, float *__restrict__ rs) {
+                         const float *__restrict__ val, float *__restrict__ sd, float *__restrict__ rs) {
   for (int row = blockIdx.x * blockDim.x + threadIdx.x; row < n; row += gridDim.x * blockDim.x) {
     const int s = row >> 6, lane = row & 63;
     const int o = sliceOff[s], K = (sliceOff[s + 1] - o) >> 6;
@@ -85,20 +88,43 @@ __global__ void kGnnDiag(int n, const int *__restrict__ sliceOff, const int *__r
       sum += val[idx];
       if (c == row) d = val[idx];
     }
-    diag[row] = d;
+    sd[row] = sqrtf(fabsf(d));
     rs[row] = d != 0.f ? sum / d : 0.f;
   }
 }
 
-// sum_i (r_i / sd_i)^2 -> scal[0] = rms
+// Graph weights in the SELL layout: a_ij / (sd_i sd_j), 0 for the diagonal
+// and padding.  Formed once per matrix: the layers read them twelve times (each
+// direction of each layer), and forming them in the layers cost a gather of
+// sd and a division per entry, repeated by the lanes that share a row.
+__global__ void kGnnWeights(int n, const int *__restrict__ sliceOff, const int *__restrict__ col,
+                            const float *__restrict__ val, const float *__restrict__ sd, float *__restrict__ ah) {
+  for (int row = blockIdx.x * blockDim.x + threadIdx.x; row < n; row += gridDim.x * blockDim.x) {
+    const int s = row >> 6, lane = row & 63;
+    const int o = sliceOff[s], K = (sliceOff[s + 1] - o) >> 6;
+    for (int e = 0; e < K; ++e) {
+      const int idx = o + (e << 6) + lane;
+      const int c = col[idx];
+      ah[idx] = (c < 0 || c == row) ? 0.f : val[idx] / (sd[row] * sd[c]);
+    }
+  }
+}
+
+// partials of sum_i (r_i / sd_i)^2; kGnnRmsFinish: scal[0] = rms
 __global__ __launch_bounds__(kRedBlock) void kGnnRms(int n, const float *__restrict__ r, const float *__restrict__ sd,
-                                                     double *scal, double *partials, unsigned *counter) {
+                                                     double *partials) {
   double d[1] = {0.};
   for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
     const double v = (double)r[i] / (double)sd[i];
     d[0] += v * v;
   }
-  if (reduceLast<1>(d, partials, counter, blockIdx.x) && threadIdx.x == 0) {
+  blockPartials<1>(d, partials, blockIdx.x);
+}
+
+__global__ __launch_bounds__(kFinBlock) void kGnnRmsFinish(int n, const double *partials, int nb, double *scal) {
+  double d[1];
+  finishPartials<1, kFinBlock>(partials, nb, d);
+  if (threadIdx.x == 0) {
     const double rms = sqrt(d[0] / (double)n);
     scal[0] = rms > 0. ? rms : 1.;
   }
@@ -124,154 +150,231 @@ __global__ void kGnnTarget(int n, const float *__restrict__ e, const float *__re
 }
 
 // ---------------------------------------------------------------- input layer
-__global__ void kGnnIn(int n, const float *__restrict__ X, const float *__restrict__ P, __bf16 *__restrict__ pre0,
-                       __bf16 *__restrict__ h0) {
-  const float *W = P;             // [4][64]
-  const float *b = P + kGnnDin * H;
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < (long)n * H; t += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(t / H), f = (int)(t % H);
-    float v = b[f];
+// h0 = relu(X W_in + b_in), eight features of a row per thread (its columns of
+// W_in in registers), and the workgroup's column sums of h0 for the first
+// layer's mean.
+__global__ __launch_bounds__(256) void kGnnIn(int n, const float *__restrict__ X, const float *__restrict__ P,
+                                              __bf16 *__restrict__ pre0, __bf16 *__restrict__ h0,
+                                              float *__restrict__ colPart) {
+  __shared__ float red[32][H + 1];
+  const int f0 = 8 * (threadIdx.x & 7), q = threadIdx.x >> 3;
+  float W[kGnnDin][8], b[8], sum[8];
 #pragma unroll
-    for (int k = 0; k < kGnnDin; ++k) v = fmaf(X[4 * i + k], W[k * H + f], v);
-    pre0[t] = (__bf16)v;
-    h0[t] = (__bf16)fmaxf(v, 0.f);
+  for (int j = 0; j < 8; ++j) {
+#pragma unroll
+    for (int k = 0; k < kGnnDin; ++k) W[k][j] = P[k * H + f0 + j];
+    b[j] = P[kGnnDin * H + f0 + j];
+    sum[j] = 0.f;
+  }
+  for (int i = blockIdx.x * 32 + q; i < n; i += gridDim.x * 32) {
+    const f32x4 x = *(const f32x4 *)&X[4 * (size_t)i];
+    bf16x8 pv, hv;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float v = b[j];
+#pragma unroll
+      for (int k = 0; k < kGnnDin; ++k) v = fmaf(x[k], W[k][j], v);
+      pv[j] = (__bf16)v;
+      hv[j] = (__bf16)fmaxf(v, 0.f);
+      sum[j] += (float)hv[j];
+    }
+    *(bf16x8 *)&pre0[(size_t)i * H + f0] = pv;
+    *(bf16x8 *)&h0[(size_t)i * H + f0] = hv;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[q][f0 + j] = sum[j];
+  __syncthreads();
+  if (threadIdx.x < H) {
+    float v = 0.f;
+    for (int k = 0; k < 32; ++k) v += red[k][threadIdx.x];
+    colPart[(size_t)blockIdx.x * H + threadIdx.x] = v;
   }
 }
 
-// ---------------------------------------------------------------- column means / sums
-// out[f] = scale * sum_i M[i][f] (M bf16 or f32 rows of 64), deterministic.
-template <class T>
-__global__ __launch_bounds__(256) void kColSum(int n, const T *__restrict__ M, float scale, float *__restrict__ out,
-                                               float *__restrict__ partials, unsigned *counter) {
-  __shared__ float red[4][H];
-  __shared__ bool last;
+// Sum over the partial records of column `col` (thread f of 64 columns, slice
+// q of 16): the calling block's 1024 threads leave the total in every thread
+// with q == 0.  Records are `stride` floats apart; the order is fixed.
+__device__ __forceinline__ float sumRecords(const float *__restrict__ partials, int records, size_t stride, int col,
+                                            bool act, float (*red)[H]) {
   const int f = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int rowsPer = (n + gridDim.x - 1) / gridDim.x;
-  const int r0 = blockIdx.x * rowsPer, r1 = min(n, r0 + rowsPer);
-  float acc = 0.f;
-  for (int i = r0 + q; i < r1; i += 4) acc += (float)M[(size_t)i * H + f];
-  red[q][f] = acc;
-  __syncthreads();
-  if (threadIdx.x < H) {
-    partials[blockIdx.x * H + f] = red[0][f] + red[1][f] + red[2][f] + red[3][f];
+  float s = 0.f;
+  for (int b0 = q; b0 < records; b0 += 16 * 8) {
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = act && b0 + 16 * u < records ? partials[(size_t)(b0 + 16 * u) * stride + col] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += t[u];
   }
-  __threadfence();
+  red[q][f] = s;
   __syncthreads();
-  if (threadIdx.x == 0) last = (atomicAdd(counter, 1u) == gridDim.x - 1);
+  float v = 0.f;
+  if (q == 0)
+    for (int k = 0; k < 16; ++k) v += red[k][f];
   __syncthreads();
-  if (!last) return;
-  __threadfence();
-  if (threadIdx.x < H) {
-    float s = 0.f;
-    for (int b = 0; b < (int)gridDim.x; ++b) s += partials[b * H + f];
-    out[f] = s * scale;
-  }
-  if (threadIdx.x == 0) *counter = 0u;
+  return v;
 }
 
-// c[f] = b[f] + sum_k g[k] Wg[k][f]
-__global__ void kGnnFold(const float *__restrict__ g, const float *__restrict__ Wg, const float *__restrict__ b,
-                         float *__restrict__ c) {
-  const int f = threadIdx.x;
-  if (f >= H) return;
-  float v = b[f];
-  for (int k = 0; k < H; ++k) v = fmaf(g[k], Wg[k * H + f], v);
-  c[f] = v;
+// g = column mean (from the partial column sums), c = b + g Wg
+__global__ __launch_bounds__(kFinThreads) void kGnnMeanFold(int n, int records, const float *__restrict__ colPart,
+                                                            const float *__restrict__ Wg, const float *__restrict__ b,
+                                                            float *__restrict__ g, float *__restrict__ c) {
+  __shared__ float red[16][H], gs[H];
+  const int f = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const float s = sumRecords(colPart, records, H, f, true, red);
+  if (q == 0) {
+    gs[f] = s * (1.f / n);
+    g[f] = gs[f];
+  }
+  __syncthreads();
+  float v = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v = fmaf(gs[4 * q + k], Wg[(4 * q + k) * H + f], v);
+  red[q][f] = v;
+  __syncthreads();
+  if (q == 0) {
+    float t = b[f];
+    for (int k = 0; k < 16; ++k) t += red[k][f];
+    c[f] = t;
+  }
 }
 
 // ---------------------------------------------------------------- message-passing layer
-// One wavefront per 16 rows: A operand = [h | A_hat h] rows (K = 128), B
-// operand = Wsm columns from LDS (stored [out col][k]).  Writes agg, pre and
-// h_new = h + relu(pre + c).
-template <class T>
-__global__ __launch_bounds__(256) void kGnnLayerFwd(int n, const __bf16 *__restrict__ h, const int *__restrict__ sliceOff,
-                                                    const int *__restrict__ col, const T *__restrict__ val,
-                                                    const float *__restrict__ sd, const __bf16 *__restrict__ wT,
+// One wavefront per 16 rows of a 64-row tile: activations [h | A_hat h]
+// (K = 128) against Wsm (LDS, stored [out col][k]).  The weights are the first
+// MFMA operand and the activations the second, with the output features dealt
+// to the weight rows so that a lane's accumulators are the features it holds as
+// an operand (8 gq + 0..7 of each half of its row): h is not read again for the
+// sum, and every access is 16 bytes of 64 contiguous ones.
+// Writes agg, pre and h_new = h + relu(pre + c); LAST also forms
+// out = h_new w_out + b_out, the other layers leave the workgroup's column
+// sums of h_new for the next layer's mean.
+// Bound by HBM: 4 x 128 B per row and the neighbours' rows out of L2.  At
+// 200,000 triangles 36.9 us (57.4 us with the graph weights formed per lane and
+// 2-byte accesses, and a separate 249 us column-sum kernel); with 8-byte
+// accesses 47.4 us.  Six wavefronts per SIMD: with the weights held in registers
+// over the tiles (196 of them, two wavefronts) 85 us.
+template <bool LAST>
+__global__ __launch_bounds__(256, 6) void kGnnLayerFwd(int n, int nTiles, int per, const __bf16 *__restrict__ h,
+                                                    const int *__restrict__ sliceOff, const int *__restrict__ col,
+                                                    const float *__restrict__ ah, const __bf16 *__restrict__ wT,
                                                     const float *__restrict__ c, __bf16 *__restrict__ agg,
-                                                    __bf16 *__restrict__ pre, __bf16 *__restrict__ hNew) {
+                                                    __bf16 *__restrict__ pre, __bf16 *__restrict__ hNew,
+                                                    float *__restrict__ colPart, const float *__restrict__ wo,
+                                                    float *__restrict__ outp) {
   __shared__ __attribute__((aligned(16))) __bf16 W[H][128 + 8];
-  __shared__ float cs[H];
+  __shared__ __attribute__((aligned(16))) float cs[H], wos[H];
+  __shared__ float red[4][H];
   for (int t = threadIdx.x; t < H * 16; t += 256) {  // 64 cols x 16 chunks of 8
     const int o = t / 16, k8 = (t % 16) * 8;
-    *(bf16x8 *)&W[o][k8] = *(const bf16x8 *)&wT[o * 128 + k8];
+    // row 16 t + m of W: feature 32 (t / 2) + 8 (m / 4) + 4 (t % 2) + m % 4
+    const int at = 16 * (2 * (o >> 5) + ((o >> 2) & 1)) + 4 * ((o >> 3) & 3) + (o & 3);
+    *(bf16x8 *)&W[at][k8] = *(const bf16x8 *)&wT[o * 128 + k8];
   }
-  if (threadIdx.x < H) cs[threadIdx.x] = c[threadIdx.x];
+  if (threadIdx.x < H) {
+    cs[threadIdx.x] = c[threadIdx.x];
+    if (LAST) wos[threadIdx.x] = wo[threadIdx.x];
+  }
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rowBase = blockIdx.x * kWgRows + wave * kRowsPerWave;
-  if (rowBase >= n) return;
-  const int r = rowBase + (lane & 15), gq = lane >> 4;
-  const bool act = r < n;
-  bf16x8 a[4];
-  // self features: chunks 0,1 ; aggregated: chunks 2,3
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, gq = lane >> 4;
+  const int group = xcdTile(blockIdx.x, gridDim.x);
+  const int t1 = min(nTiles, (group + 1) * per);
+  f32x4 sum[4];
 #pragma unroll
-  for (int kc = 0; kc < 2; ++kc) {
-    const int f0 = 32 * kc + 8 * gq;
-    if (act) a[kc] = *(const bf16x8 *)&h[(size_t)r * H + f0];
-    else
-      for (int j = 0; j < 8; ++j) a[kc][j] = (__bf16)0.f;
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (act) {
-      const int s = r >> 6, l = r & 63;
-      const int o = sliceOff[s], K = (sliceOff[s + 1] - o) >> 6;
-      for (int e = 0; e < K; ++e) {
-        int cc;
-        const float w = ahat(col, val, sd, o + (e << 6) + l, r, cc);
-        if (w == 0.f) continue;
-        const bf16x8 hv = *(const bf16x8 *)&h[(size_t)cc * H + f0];
+  for (int t = 0; t < 4; ++t) sum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int tile = group * per; tile < t1; ++tile) {
+    const int l = 16 * wave + (lane & 15), r = tile * kTileRows + l;
+    const bool act = r < n;
+    const int o = sliceOff[tile], K = act ? (sliceOff[tile + 1] - o) >> 6 : 0;
+    const size_t at = (size_t)(act ? r : 0) * H;
+    const bf16x8 zero = {};
+    bf16x8 a[4];
+    // one half of the features at a time (both halves' sums and neighbours'
+    // rows together hold 40 more registers); the columns and weights come from
+    // L1 the second time
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] = fmaf(w, (float)hv[j], acc[j]);
+    for (int kc = 0; kc < 2; ++kc) {
+      asm volatile("" ::: "memory");
+      const int f0 = 32 * kc + 8 * gq;
+      a[kc] = act ? *(const bf16x8 *)&h[at + f0] : zero;
+      float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (int e0 = 0; e0 < K; e0 += 4) {
+        int cc[4];
+        float w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool in = e0 + q < K;
+          const int idx = o + ((e0 + (in ? q : 0)) << 6) + l;
+          cc[q] = col[idx];
+          w[q] = in ? ah[idx] : 0.f;
+        }
+        bf16x8 x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = w[q] != 0.f ? *(const bf16x8 *)&h[(size_t)cc[q] * H + f0] : zero;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[j] = fmaf(w[q], (float)x[q][j], acc[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[2 + kc][j] = (__bf16)acc[j];
+      if (act) *(bf16x8 *)&agg[at + f0] = a[2 + kc];
+    }
+    // lane: row r, half kc, features 32 kc + 8 gq + 4 u + v
+    float dot = 0.f;
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      asm volatile("" ::: "memory");  // this half's weights are read here, not held
+      const int f0 = 32 * kc + 8 * gq;
+      bf16x8 pv, hv;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        f32x4 out = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4)
+          out = mfma(*(const bf16x8 *)&W[16 * (2 * kc + u) + (lane & 15)][32 * c4 + 8 * gq], a[c4], out);
+        const f32x4 cv = *(const f32x4 *)&cs[f0 + 4 * u];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float p = out[v] + cv[v];
+          const __bf16 hn = (__bf16)((float)a[kc][4 * u + v] + fmaxf(p, 0.f));
+          pv[4 * u + v] = (__bf16)p;
+          hv[4 * u + v] = hn;
+          if (!LAST) sum[2 * kc + u][v] += act ? (float)hn : 0.f;
+          if (LAST) dot = fmaf((float)hn, wos[f0 + 4 * u + v], dot);
+        }
+      }
+      if (act) {
+        *(bf16x8 *)&pre[at + f0] = pv;
+        *(bf16x8 *)&hNew[at + f0] = hv;
       }
     }
-    bf16x8 av;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) av[j] = (__bf16)acc[j];
-    a[2 + kc] = av;
-    if (act) *(bf16x8 *)&agg[(size_t)r * H + f0] = av;
-  }
-  f32x4 out[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    out[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int oc = 16 * t + (lane & 15);
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-      const bf16x8 b = *(const bf16x8 *)&W[oc][32 * kc + 8 * gq];
-      out[t] = mfma(a[kc], b, out[t]);
+    if (LAST) {
+      dot += __shfl_xor(dot, 16, 64);
+      dot += __shfl_xor(dot, 32, 64);
+      if (act && gq == 0) outp[r] = dot + wo[H];
     }
   }
-  // D layout: row = 4*gq + v, col = 16*t + lane%16
+  if (!LAST) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int oc = 16 * t + (lane & 15);
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = rowBase + 4 * gq + v;
-      if (row < n) {
-        const float p = out[t][v] + cs[oc];
-        pre[(size_t)row * H + oc] = (__bf16)p;
-        hNew[(size_t)row * H + oc] = (__bf16)((float)h[(size_t)row * H + oc] + fmaxf(p, 0.f));
+      for (int v = 0; v < 4; ++v) {
+        float x = sum[t][v];
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) x += __shfl_xor(x, m, 64);
+        if ((lane & 15) == 0) red[wave][32 * (t >> 1) + 8 * gq + 4 * (t & 1) + v] = x;
       }
-    }
+    __syncthreads();
+    if (threadIdx.x < H)
+      colPart[(size_t)blockIdx.x * H + threadIdx.x] =
+          red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
   }
 }
 
-// ---------------------------------------------------------------- output layer
-// out_i = h_i . w_out + b_out
-__global__ __launch_bounds__(256) void kGnnOut(int n, const __bf16 *__restrict__ h, const float *__restrict__ wo,
-                                               float *__restrict__ out) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    float v = wo[H];
-    for (int f = 0; f < H; ++f) v = fmaf((float)h[(size_t)i * H + f], wo[f], v);
-    out[i] = v;
-  }
-}
-
-// a = out.t, p = |out|^2, q = |t|^2 ; loss = 1 - a^2/(p q) -> scal[1..4];
-// scal[5] accumulates losses over training steps
+// a = out.t, p = |out|^2, q = |t|^2 (partials); kGnnLossFinish: loss =
+// 1 - a^2/(p q) -> scal[1..4]; scal[5] accumulates losses over training steps
 __global__ __launch_bounds__(kRedBlock) void kGnnLossCos(int n, const float *__restrict__ out,
-                                                         const float *__restrict__ t, double *scal,
-                                                         double *partials, unsigned *counter) {
+                                                         const float *__restrict__ t, double *partials) {
   double d[3] = {0., 0., 0.};
   for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
     const double o = out[i], ti = t[i];
@@ -279,7 +382,13 @@ __global__ __launch_bounds__(kRedBlock) void kGnnLossCos(int n, const float *__r
     d[1] += o * o;
     d[2] += ti * ti;
   }
-  if (reduceLast<3>(d, partials, counter, blockIdx.x) && threadIdx.x == 0) {
+  blockPartials<3>(d, partials, blockIdx.x);
+}
+
+__global__ __launch_bounds__(kFinBlock) void kGnnLossFinish(const double *partials, int nb, double *scal) {
+  double d[3];
+  finishPartials<3, kFinBlock>(partials, nb, d);
+  if (threadIdx.x == 0) {
     const double pq = d[1] * d[2];
     const double loss = pq > 0. ? 1.0 - d[0] * d[0] / pq : 1.0;
     scal[1] = loss;
@@ -290,19 +399,14 @@ __global__ __launch_bounds__(kRedBlock) void kGnnLossCos(int n, const float *__r
   }
 }
 
-// dout_i = 2a/(p q) (a out_i / p - t_i) ; dh_L = dout w_out^T
+// dout_i = 2a/(p q) (a out_i / p - t_i)
 __global__ void kGnnDout(int n, const float *__restrict__ out, const float *__restrict__ t,
-                         const float *__restrict__ wo, const double *__restrict__ scal, float *__restrict__ dout,
-                         float *__restrict__ dh) {
+                         const double *__restrict__ scal, float *__restrict__ dout) {
   const double a = scal[2], p = scal[3], q = scal[4];
   const bool ok = p > 0. && q > 0.;
   const float c1 = ok ? (float)(2.0 * a / (p * q)) : 0.f, c2 = ok ? (float)(a / p) : 0.f;
-  for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < (long)n * H; k += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(k / H), f = (int)(k % H);
-    const float d = c1 * (c2 * out[i] - t[i]);
-    if (f == 0) dout[i] = d;
-    dh[k] = d * wo[f];
-  }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    dout[i] = c1 * (c2 * out[i] - t[i]);
 }
 
 // residual objective: c = out / sd
@@ -319,222 +423,304 @@ __global__ void kGnnResDq(int n, const float *__restrict__ q, const float *__res
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dq[i] = c1 * (c2 * q[i] - r[i]);
 }
 
-// residual objective: dout_i = g_i / sd_i (g = A dq) ; dh_L = dout w_out^T
+// residual objective: dout_i = g_i / sd_i (g = A dq)
 __global__ void kGnnResDout(int n, const float *__restrict__ g, const float *__restrict__ sd,
-                            const float *__restrict__ wo, float *__restrict__ dout, float *__restrict__ dh) {
-  for (long k = blockIdx.x * (long)blockDim.x + threadIdx.x; k < (long)n * H; k += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(k / H), f = (int)(k % H);
-    const float d = g[i] / sd[i];
-    if (f == 0) dout[i] = d;
-    dh[k] = d * wo[f];
-  }
+                            float *__restrict__ dout) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dout[i] = g[i] / sd[i];
 }
 
-// grad of w_out / b_out: per-block partials of h^T dout and sum(dout)
+// grad of w_out / b_out: per-workgroup partials of h^T dout and sum(dout),
+// eight features of a row per thread
 __global__ __launch_bounds__(256) void kGnnOutGrad(int n, const __bf16 *__restrict__ h, const float *__restrict__ dout,
                                                    float *__restrict__ partials) {
-  __shared__ float red[4][H + 1];
-  const int f = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int rowsPer = (n + gridDim.x - 1) / gridDim.x;
-  const int r0 = blockIdx.x * rowsPer, r1 = min(n, r0 + rowsPer);
-  float acc = 0.f, accb = 0.f;
-  for (int i = r0 + q; i < r1; i += 4) {
+  __shared__ float red[32][H + 1];
+  const int f0 = 8 * (threadIdx.x & 7), q = threadIdx.x >> 3;
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, accb = 0.f;
+  for (int i = blockIdx.x * 32 + q; i < n; i += gridDim.x * 32) {
     const float d = dout[i];
-    acc = fmaf((float)h[(size_t)i * H + f], d, acc);
-    if (f == 0) accb += d;
+    const bf16x8 hv = *(const bf16x8 *)&h[(size_t)i * H + f0];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)hv[j], d, acc[j]);
+    accb += d;
   }
-  red[q][f] = acc;
-  if (f == 0) red[q][H] = accb;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[q][f0 + j] = acc[j];
+  if (f0 == 0) red[q][H] = accb;
   __syncthreads();
   if (threadIdx.x < H + 1) {
-    const int k = threadIdx.x;
-    partials[blockIdx.x * (H + 1) + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    float v = 0.f;
+    for (int k = 0; k < 32; ++k) v += red[k][threadIdx.x];
+    partials[(size_t)blockIdx.x * (H + 1) + threadIdx.x] = v;
   }
 }
 
-// ---------------------------------------------------------------- backward, data part
-// dpre = dh * (pre > 0) ; dSA[r][k] = sum_c dpre[r][c] W[k][c]  (k < 128)
-__global__ __launch_bounds__(256) void kGnnBwdData(int n, const float *__restrict__ dh, const __bf16 *__restrict__ pre,
-                                                   const __bf16 *__restrict__ wN, __bf16 *__restrict__ dpre,
-                                                   float *__restrict__ dSA) {
-  __shared__ __attribute__((aligned(16))) __bf16 W[128][H + 8];
+// ---------------------------------------------------------------- backward layer
+// Rows of a feature, eight to a 16-byte chunk: chunk `chunk` (of 8) of feature
+// f in a transposed tile of 64 rows.  Pitch 72 elements and the chunk index
+// xored with f / 8 keep both the packed 4-byte writes (eight features of one
+// row pair per instruction step) and the 16-byte reads (16 neighbouring
+// features) free of bank conflicts.
+constexpr int kTPitch = 72;
+__device__ __forceinline__ int tileAt(int f, int chunk) { return f * kTPitch + ((chunk ^ ((f >> 3) & 7)) << 3); }
+
+// Backward pass of one layer over the workgroup's tiles:
+//   dh    = FIRST ? dout w_out^T : dhIn + gterm + A_hat^T daggIn   (A_hat symmetric)
+//   dpre  = dh * (pre > 0)
+//   dhOut = dh + dpre Ws^T, daggOut = dpre Wm^T                    (FP32)
+//   partials of dWsm = [h | agg]^T dpre and db = column sums of dpre
+// The combination with the layer above (dhIn, daggIn, gterm) is formed as it is
+// read, and dpre stays in registers and LDS, so per row the kernel moves
+// 7 x 128 B to and from HBM (dh, pre, h, agg in; dh, dagg in FP32 out) and the
+// neighbours' dagg rows out of L2.  MFMA operands: the data product takes the
+// weights first and dpre second, the output features dealt to the weight rows
+// as in the forward layer: a lane holds the same 16 features of its row in dh,
+// dpre and the products.  The
+// weight product contracts over rows: both operands go through LDS transposed,
+// two rows packed per 4-byte write.
+// At 200,000 triangles 79 us per layer, 3.6 TB/s; as three kernels 66.7 us
+// (data product), 637 us (weight product: 98 workgroups, 2-byte transposed
+// writes) and 116 us (combination).
+template <bool FIRST>
+__global__ __launch_bounds__(256) void kGnnLayerBwd(
+    int n, int nTiles, int per, const float *__restrict__ dout, const float *__restrict__ wo, const float *dhIn,
+    const float *__restrict__ daggIn, const float *__restrict__ gterm, const int *__restrict__ sliceOff,
+    const int *__restrict__ col, const float *__restrict__ ah, const __bf16 *__restrict__ pre,
+    const __bf16 *__restrict__ h, const __bf16 *__restrict__ agg, const __bf16 *__restrict__ wN, float *dhOut,
+    float *__restrict__ daggOut, float *__restrict__ partials) {
+  __shared__ __attribute__((aligned(16))) __bf16 W[128][H + 8];  // [k][c]
+  __shared__ __attribute__((aligned(16))) __bf16 HA[128 * kTPitch], DP[H * kTPitch];
+  __shared__ __attribute__((aligned(16))) float fs[H];           // FIRST: w_out, else gterm
   for (int t = threadIdx.x; t < 128 * 8; t += 256) {
-    const int k = t / 8, c8 = (t % 8) * 8;
-    *(bf16x8 *)&W[k][c8] = *(const bf16x8 *)&wN[k * H + c8];
+    const int k = t >> 3, c8 = 8 * (t & 7);
+    // row 16 t + m of W: feature 32 (t / 2) + 8 (m / 4) + 4 (t % 2) + m % 4
+    const int at = 16 * (2 * (k >> 5) + ((k >> 2) & 1)) + 4 * ((k >> 3) & 3) + (k & 3);
+    *(bf16x8 *)&W[at][c8] = *(const bf16x8 *)&wN[k * H + c8];
   }
-  __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rowBase = blockIdx.x * kWgRows + wave * kRowsPerWave;
-  if (rowBase >= n) return;
-  const int r = rowBase + (lane & 15), gq = lane >> 4;
-  const bool act = r < n;
-  bf16x8 a[2];
-#pragma unroll
-  for (int kc = 0; kc < 2; ++kc) {
-    const int f0 = 32 * kc + 8 * gq;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = 0.f;
-      if (act) {
-        const size_t idx = (size_t)r * H + f0 + j;
-        v = (float)pre[idx] > 0.f ? dh[idx] : 0.f;
-      }
-      a[kc][j] = (__bf16)v;
-    }
-    if (act) *(bf16x8 *)&dpre[(size_t)r * H + f0] = a[kc];
-  }
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int k = 16 * t + (lane & 15);
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) acc = mfma(a[kc], *(const bf16x8 *)&W[k][32 * kc + 8 * gq], acc);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = rowBase + 4 * gq + v;
-      if (row < n) dSA[(size_t)row * 128 + k] = acc[v];
-    }
-  }
-}
-
-// ---------------------------------------------------------------- backward, weight part
-// Per workgroup partial of dWsm[k][c] = sum_r [h | agg][r][k] dpre[r][c] over
-// kChunkRows rows (MFMA with K = rows), and of db[c] = sum_r dpre[r][c].
-// Wave w owns k in [32w, 32w+32) (two 16-row tiles) x 4 column tiles.
-__global__ __launch_bounds__(256) void kGnnBwdWeights(int n, const __bf16 *__restrict__ h,
-                                                      const __bf16 *__restrict__ agg,
-                                                      const __bf16 *__restrict__ dpre, float *__restrict__ partials) {
-  __shared__ __attribute__((aligned(16))) __bf16 HA[128][32 + 8];  // [feature][row]
-  __shared__ __attribute__((aligned(16))) __bf16 DP[H][32 + 8];    // [col][row]
-  __shared__ float dbs[4][H];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, gq = lane >> 4;
-  const int r0 = blockIdx.x * kChunkRows, r1 = min(n, r0 + kChunkRows);
+  if (threadIdx.x < H) fs[threadIdx.x] = FIRST ? wo[threadIdx.x] : gterm[threadIdx.x];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, gq = lane >> 4, l16 = lane & 15;
+  auto feat = [&](int t) { return 32 * (t >> 1) + 8 * gq + 4 * (t & 1); };  // first feature of dh[t]
+  const int group = xcdTile(blockIdx.x, gridDim.x);
+  const int t1 = min(nTiles, (group + 1) * per);
   f32x4 acc[2][4];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float dbAcc = 0.f;
-  for (int base = r0; base < r1; base += 32) {
-    __syncthreads();
-    // stage 32 rows, transposed
-    for (int t = threadIdx.x; t < 32 * 128; t += 256) {
-      const int rr = t / 128, k = t % 128, row = base + rr;
-      __bf16 v = (__bf16)0.f;
-      if (row < r1) v = k < H ? h[(size_t)row * H + k] : agg[(size_t)row * H + (k - H)];
-      HA[k][rr] = v;
-    }
-    for (int t = threadIdx.x; t < 32 * H; t += 256) {
-      const int rr = t / H, cc = t % H, row = base + rr;
-      DP[cc][rr] = row < r1 ? dpre[(size_t)row * H + cc] : (__bf16)0.f;
-    }
-    __syncthreads();
-    {
-      // column sums of dpre for db: thread (q, c) sums 8 rows
-      const int cc = threadIdx.x & 63, q = threadIdx.x >> 6;
-      for (int rr = q * 8; rr < q * 8 + 8; ++rr) dbAcc += (float)DP[cc][rr];
-    }
+  float db = 0.f;
+  for (int tile = group * per; tile < t1; ++tile) {
+    __syncthreads();  // the previous tile's LDS reads are done (first tile: W and fs are written)
+    const int base = tile * kTileRows;
+    // stage [h | agg]^T: row pair rp, octet of features o8 (0..15)
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const int k = 32 * wave + 16 * a + (lane & 15);
-      const bf16x8 av = *(const bf16x8 *)&HA[k][8 * gq];
+    for (int it = 0; it < 2; ++it) {
+      const int item = threadIdx.x + 256 * it;
+      const int o8 = item & 15, rp = item >> 4;
+      const int row = base + 2 * rp;
+      const __bf16 *src = o8 < 8 ? h : agg;
+      const int f0 = 8 * (o8 & 7);
+      bf16x8 u = {}, v = {};
+      if (row < n) u = *(const bf16x8 *)&src[(size_t)row * H + f0];
+      if (row + 1 < n) v = *(const bf16x8 *)&src[(size_t)(row + 1) * H + f0];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int cc = 16 * t + (lane & 15);
-        acc[a][t] = mfma(av, *(const bf16x8 *)&DP[cc][8 * gq], acc[a][t]);
+      for (int j = 0; j < 8; ++j) {
+        typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+        *(bf16x2 *)&HA[tileAt(8 * o8 + j, rp >> 2) + 2 * (rp & 3)] = bf16x2{u[j], v[j]};
       }
     }
+    const int l = 16 * wave + l16, r = base + l;
+    const bool act = r < n;
+    const size_t at = (size_t)(act ? r : 0) * H;
+    f32x4 dh[4];
+    if (FIRST) {
+      const float d = act ? dout[r] : 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) dh[t] = d * *(const f32x4 *)&fs[feat(t)];
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) dh[t] = *(const f32x4 *)&dhIn[at + feat(t)] + *(const f32x4 *)&fs[feat(t)];
+      const int o = sliceOff[tile], K = act ? (sliceOff[tile + 1] - o) >> 6 : 0;
+      for (int e0 = 0; e0 < K; e0 += 2) {
+        int cc[2];
+        float w[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const bool in = e0 + q < K;
+          const int idx = o + ((e0 + (in ? q : 0)) << 6) + l;
+          cc[q] = col[idx];
+          w[q] = in ? ah[idx] : 0.f;
+        }
+        f32x4 x[2][4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            x[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (w[q] != 0.f) x[q][t] = *(const f32x4 *)&daggIn[(size_t)cc[q] * H + feat(t)];
+          }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dh[t][v] = fmaf(w[q], x[q][t][v], dh[t][v]);
+      }
+    }
+    bf16x8 a[2];
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const bf16x8 pv = *(const bf16x8 *)&pre[at + 32 * kc + 8 * gq];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[kc][j] = (__bf16)(act && (float)pv[j] > 0.f ? dh[2 * kc + (j >> 2)][j & 3] : 0.f);
+    }
+    // dpre^T: lanes of rows r, r ^ 1 exchange halves and write row pairs; the
+    // even row writes the features of kc = 0, the odd row those of kc = 1
+    {
+      typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+      const u32x4 w0 = __builtin_bit_cast(u32x4, a[0]), w1 = __builtin_bit_cast(u32x4, a[1]);
+      const bool odd = lane & 1;
+      const int rp = l >> 1;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const unsigned got = __shfl_xor(odd ? w0[m] : w1[m], 1, 64);
+        const unsigned lo = odd ? got : w0[m], hi = odd ? w1[m] : got;  // row pair's even / odd row
+        // word m: features j = 2 m, 2 m + 1 of the half
+        const int f = (odd ? 32 : 0) + 8 * gq + 2 * m;
+        *(unsigned *)&DP[tileAt(f, rp >> 2) + 2 * (rp & 3)] = (lo & 0xffffu) | (hi << 16);
+        *(unsigned *)&DP[tileAt(f + 1, rp >> 2) + 2 * (rp & 3)] = (lo >> 16) | (hi & 0xffff0000u);
+      }
+    }
+    // data product
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      f32x4 p = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) p = mfma(*(const bf16x8 *)&W[16 * t + l16][32 * kc + 8 * gq], a[kc], p);
+      if (act) {
+        if (t < 4) *(f32x4 *)&dhOut[at + feat(t)] = dh[t & 3] + p;
+        else *(f32x4 *)&daggOut[at + feat(t - 4)] = p;
+      }
+    }
+    __syncthreads();
+    // weight product: wave w owns k in [32 w, 32 w + 32)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      bf16x8 av[2], bv[4];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) av[q] = *(const bf16x8 *)&HA[tileAt(32 * wave + 16 * q + l16, 4 * kk + gq)];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) bv[t] = *(const bf16x8 *)&DP[tileAt(16 * t + l16, 4 * kk + gq)];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[q][t] = mfma(av[q], bv[t], acc[q][t]);
+      const bf16x8 mine = *(const bf16x8 *)&DP[tileAt(16 * wave + l16, 4 * kk + gq)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) db += (float)mine[j];
+    }
   }
-  // partial layout per block: [128][64] dW then [64] db
+  // partial record: [128][64] dW then [64] db
   float *P = partials + (size_t)blockIdx.x * (128 * H + H);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int q = 0; q < 2; ++q)
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int k = 32 * wave + 16 * a + 4 * gq + v;
-        const int cc = 16 * t + (lane & 15);
-        P[k * H + cc] = acc[a][t][v];
-      }
+      for (int v = 0; v < 4; ++v) P[(32 * wave + 16 * q + 4 * gq + v) * H + 16 * t + l16] = acc[q][t][v];
+  db += __shfl_xor(db, 16, 64);
+  db += __shfl_xor(db, 32, 64);
+  if (gq == 0) P[128 * H + 16 * wave + l16] = db;
+}
+
+// grad[k] = sum of the partial records' entry k (fixed order), 64 entries per block
+__global__ __launch_bounds__(kFinThreads) void kSumPartials(int records, int m, const float *__restrict__ partials,
+                                                            float *__restrict__ grad) {
+  __shared__ float red[16][H];
+  const int k = blockIdx.x * H + (threadIdx.x & 63);
+  const float v = sumRecords(partials, records, m, k, k < m, red);
+  if (threadIdx.x < H && k < m) grad[k] = v;
+}
+
+// The sums of a backward layer's records: dWsm (blocks 0 to 127) and db (block
+// 128), which then also gives dWg[k][c] = g[k] db[c] and
+// gterm[k] = sum_c Wg[k][c] db[c] / n.
+__global__ __launch_bounds__(kFinThreads) void kGnnSumLayer(int n, int records, const float *__restrict__ partials,
+                                                            const float *__restrict__ g, const float *__restrict__ Wg,
+                                                            float *__restrict__ dWsm, float *__restrict__ db,
+                                                            float *__restrict__ dWg, float *__restrict__ gterm) {
+  __shared__ float red[16][H], dbs[H];
+  const int f = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int k = blockIdx.x * H + f;
+  const float v = sumRecords(partials, records, 128 * H + H, k, true, red);
+  if (blockIdx.x < 128) {
+    if (q == 0) dWsm[k] = v;
+    return;
+  }
+  if (q == 0) {
+    db[f] = v;
+    dbs[f] = v;
+  }
   __syncthreads();
-  dbs[threadIdx.x >> 6][threadIdx.x & 63] = dbAcc;
-  __syncthreads();
-  if (threadIdx.x < H) P[128 * H + threadIdx.x] = dbs[0][threadIdx.x] + dbs[1][threadIdx.x] + dbs[2][threadIdx.x] + dbs[3][threadIdx.x];
-}
-
-// Sum per-block partials (fixed order) into grad[dst .. dst+m)
-__global__ void kSumPartials(int nBlocks, int m, const float *__restrict__ partials, float *__restrict__ grad) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < m; k += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int b = 0; b < nBlocks; ++b) s += partials[(size_t)b * m + k];
-    grad[k] = s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = 4 * q + j;
+    dWg[row * H + f] = g[row] * dbs[f];
+    float s = Wg[row * H + f] * dbs[f];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (f == 0) gterm[row] = s / (float)n;
   }
 }
 
-// As kSumPartials with the record split: k < split -> dst1[k], else dst2[k - split]
-__global__ void kSumPartialsStrided(int nBlocks, int m, const float *__restrict__ partials, float *__restrict__ dst1,
-                                    int split, float *__restrict__ dst2) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < m; k += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int b = 0; b < nBlocks; ++b) s += partials[(size_t)b * m + k];
-    if (k < split) dst1[k] = s;
-    else dst2[k - split] = s;
-  }
-}
-
-// dWg[k][c] = g[k] * db[c]; gterm[k] = sum_c Wg[k][c] db[c] / n
-__global__ void kGnnGlobalGrad(int n, const float *__restrict__ g, const float *__restrict__ db,
-                               const float *__restrict__ Wg, float *__restrict__ dWg, float *__restrict__ gterm) {
-  const int k = threadIdx.x;
-  if (k >= H) return;
-  float s = 0.f;
-  for (int c = 0; c < H; ++c) {
-    dWg[k * H + c] = g[k] * db[c];
-    s = fmaf(Wg[k * H + c], db[c], s);
-  }
-  gterm[k] = s / (float)n;
-}
-
-// dh_prev = dh + dself + A_hat^T dagg + gterm   (A_hat symmetric)
-template <class T>
-__global__ void kGnnBwdCombine(int n, float *__restrict__ dh, const float *__restrict__ dSA,
-                               const int *__restrict__ sliceOff, const int *__restrict__ col, const T *__restrict__ val,
-                               const float *__restrict__ sd, const float *__restrict__ gterm) {
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < (long)n * H; t += (long)gridDim.x * blockDim.x) {
-    const int r = (int)(t / H), f = (int)(t % H);
-    float v = dh[t] + dSA[(size_t)r * 128 + f] + gterm[f];
-    const int s = r >> 6, l = r & 63;
+// input layer gradient partials: dW_in[k][c] = sum_r X[r][k] dpre0[r][c],
+// db_in[c], with dh0 = dhIn + gterm + A_hat^T dagg of the first layer formed
+// as it is read: four features of a row per thread, 16 rows per step
+__global__ __launch_bounds__(256) void kGnnInGrad(int n, const float *__restrict__ X, const __bf16 *__restrict__ pre0,
+                                                  const float *__restrict__ dhIn, const float *__restrict__ dagg,
+                                                  const float *__restrict__ gterm, const int *__restrict__ sliceOff,
+                                                  const int *__restrict__ col, const float *__restrict__ ah,
+                                                  float *__restrict__ partials) {
+  __shared__ float red[16][H];
+  const int f0 = 4 * (threadIdx.x & 15), q = threadIdx.x >> 4;
+  const f32x4 g = *(const f32x4 *)&gterm[f0];
+  f32x4 acc[kGnnDin + 1];
+#pragma unroll
+  for (int k = 0; k <= kGnnDin; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int b = xcdTile(blockIdx.x, gridDim.x); b * 16 < n; b += gridDim.x) {
+    const int i = b * 16 + q;
+    if (i >= n) continue;
+    const size_t at = (size_t)i * H + f0;
+    f32x4 dh = *(const f32x4 *)&dhIn[at] + g;
+    const int s = i >> 6, l = i & 63;
     const int o = sliceOff[s], K = (sliceOff[s + 1] - o) >> 6;
     for (int e = 0; e < K; ++e) {
-      int cc;
-      const float w = ahat(col, val, sd, o + (e << 6) + l, r, cc);
-      if (w != 0.f) v = fmaf(w, dSA[(size_t)cc * 128 + H + f], v);
+      const int idx = o + (e << 6) + l;
+      const float w = ah[idx];
+      if (w == 0.f) continue;
+      const f32x4 x = *(const f32x4 *)&dagg[(size_t)col[idx] * H + f0];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dh[v] = fmaf(w, x[v], dh[v]);
     }
-    dh[t] = v;
-  }
-}
-
-// input layer gradient partials: dW_in[k][c] = sum_r X[r][k] dpre0[r][c], db_in[c]
-__global__ __launch_bounds__(256) void kGnnInGrad(int n, const float *__restrict__ X, const __bf16 *__restrict__ pre0,
-                                                  const float *__restrict__ dh, float *__restrict__ partials) {
-  __shared__ float red[4][(kGnnDin + 1) * H];
-  const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int rowsPer = (n + gridDim.x - 1) / gridDim.x;
-  const int r0 = blockIdx.x * rowsPer, r1 = min(n, r0 + rowsPer);
-  float acc[kGnnDin + 1] = {0, 0, 0, 0, 0};
-  for (int i = r0 + q; i < r1; i += 4) {
-    const size_t idx = (size_t)i * H + c;
-    const float dp = (float)pre0[idx] > 0.f ? dh[idx] : 0.f;
+    const bf16x4 pv = *(const bf16x4 *)&pre0[at];
+    const f32x4 x = *(const f32x4 *)&X[4 * (size_t)i];
 #pragma unroll
-    for (int k = 0; k < kGnnDin; ++k) acc[k] = fmaf(X[4 * i + k], dp, acc[k]);
-    acc[kGnnDin] += dp;
+    for (int v = 0; v < 4; ++v) {
+      const float dp = (float)pv[v] > 0.f ? dh[v] : 0.f;
+#pragma unroll
+      for (int k = 0; k < kGnnDin; ++k) acc[k][v] = fmaf(x[k], dp, acc[k][v]);
+      acc[kGnnDin][v] += dp;
+    }
   }
 #pragma unroll
-  for (int k = 0; k <= kGnnDin; ++k) red[q][k * H + c] = acc[k];
-  __syncthreads();
-  for (int t = threadIdx.x; t < (kGnnDin + 1) * H; t += 256)
-    partials[(size_t)blockIdx.x * (kGnnDin + 1) * H + t] = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+  for (int k = 0; k <= kGnnDin; ++k) {
+    *(f32x4 *)&red[q][f0] = acc[k];
+    __syncthreads();
+    if (threadIdx.x < H) {
+      float v = 0.f;
+      for (int j = 0; j < 16; ++j) v += red[j][threadIdx.x];
+      partials[(size_t)blockIdx.x * (kGnnDin + 1) * H + k * H + threadIdx.x] = v;
+    }
+    __syncthreads();
+  }
 }
 
 // Adam (Kingma & Ba 2015), then refresh the BF16 weight copies
@@ -612,29 +798,29 @@ void ensureNet(phase_hip_solver *s) {
     G.agg.alloc((size_t)L * n * H);
     G.pre.alloc((size_t)L * n * H);
     G.pre0.alloc((size_t)n * H);
-    G.dpre.alloc((size_t)n * H);
     G.dh.alloc((size_t)n * H);
-    G.dSA.alloc((size_t)n * 128);
+    G.dagg.alloc(2 * (size_t)n * H);
     G.gmean.alloc((size_t)L * H);
     G.cvec.alloc((size_t)L * H);
-    const int nbW = (n + kChunkRows - 1) / kChunkRows;
-    G.partials.alloc(std::max<size_t>((size_t)nbW * (128 * H + H), (size_t)2048 * (kGnnDin + 1) * H));
+    G.partials.alloc(std::max<size_t>((size_t)tilesFor(n, kBwdGroups).groups * (128 * H + H),
+                                      (size_t)kFwdGroups * (kGnnDin + 1) * H));
     G.scal.alloc(8);
     G.scal.zero(s->stream);
-    G.counter.alloc(1);
-    G.counter.zero(s->stream);
     G.wT.alloc((size_t)L * 128 * H);
     G.wN.alloc((size_t)L * 128 * H);
   }
 }
 
-// Graph quantities of the current matrix (FP32 SELL copy): sd, row-sum ratio.
+// Graph quantities of the current matrix (FP32 SELL copy): sd, row-sum ratio,
+// graph weights.
 void prepareGraph(phase_hip_solver *s) {
   GnnState &G = *s->gnn;
   const int n = s->rank;
+  G.ahat.alloc(s->dSell32.n);
   hipLaunchKernelGGL(kGnnDiag, dim3(g1(n)), dim3(256), 0, s->stream, n, s->dSliceOff.p, s->dSellCol.p, s->dSell32.p,
-                     G.dOut.p, G.rowsum.p);
-  hipLaunchKernelGGL(kGnnScale, dim3(g1(n)), dim3(256), 0, s->stream, n, G.dOut.p, G.rowsum.p, G.sd.p, G.rowsum.p);
+                     G.sd.p, G.rowsum.p);
+  hipLaunchKernelGGL(kGnnWeights, dim3(g1(n)), dim3(256), 0, s->stream, n, s->dSliceOff.p, s->dSellCol.p,
+                     s->dSell32.p, G.sd.p, G.ahat.p);
 }
 
 void castWeights(phase_hip_solver *s) {
@@ -649,8 +835,9 @@ __bf16 *hL(GnnState &G, int l) { return G.h.p + (size_t)l * G.n * H; }
 void gnnFeatures(phase_hip_solver *s, const float *r, const float *z) {
   GnnState &G = *s->gnn;
   const int n = s->rank;
-  hipLaunchKernelGGL(kGnnRms, dim3(gridFor1(n)), dim3(kRedBlock), 0, s->stream, n, r, G.sd.p, G.scal.p, s->dPartials.p,
-                     s->dCounter.p);
+  const int gr = gridFor1(n);
+  hipLaunchKernelGGL(kGnnRms, dim3(gr), dim3(kRedBlock), 0, s->stream, n, r, G.sd.p, s->dPartials.p);
+  hipLaunchKernelGGL(kGnnRmsFinish, dim3(1), dim3(kFinBlock), 0, s->stream, n, s->dPartials.p, gr, G.scal.p);
   hipLaunchKernelGGL(kGnnFeatures, dim3(g1(n)), dim3(256), 0, s->stream, n, r, z, G.sd.p, G.rowsum.p, G.scal.p, G.X.p);
 }
 
@@ -662,48 +849,45 @@ void gnnForward(phase_hip_solver *s) {
   GnnState &G = *s->gnn;
   const int n = s->rank, L = G.lay.L;
   const float *P = G.params.p;
-  hipLaunchKernelGGL(kGnnIn, dim3(g1((long)n * H)), dim3(256), 0, s->stream, n, G.X.p, P + G.lay.inW(), G.pre0.p,
-                     hL(G, 0));
-  const int nwg = (n + kWgRows - 1) / kWgRows;
-  const int ncs = std::min(1024, std::max(1, (n + 255) / 256));
+  const Tiles T = tilesFor(n, kFwdGroups);
+  int records = std::min(kFwdGroups, std::max(1, (n + 31) / 32));
+  hipLaunchKernelGGL(kGnnIn, dim3(records), dim3(256), 0, s->stream, n, G.X.p, P + G.lay.inW(), G.pre0.p, hL(G, 0),
+                     G.partials.p);
   for (int l = 0; l < L; ++l) {
-    hipLaunchKernelGGL((kColSum<__bf16>), dim3(ncs), dim3(256), 0, s->stream, n, (const __bf16 *)hL(G, l), 1.f / n,
-                       G.gmean.p + l * H, G.partials.p, G.counter.p);
-    hipLaunchKernelGGL(kGnnFold, dim3(1), dim3(64), 0, s->stream, G.gmean.p + l * H, P + G.lay.wg(l), P + G.lay.b(l),
-                       G.cvec.p + l * H);
-    hipLaunchKernelGGL((kGnnLayerFwd<float>), dim3(nwg), dim3(256), 0, s->stream, n, (const __bf16 *)hL(G, l),
-                       s->dSliceOff.p, s->dSellCol.p, s->dSell32.p, G.sd.p, G.wT.p + (size_t)l * 128 * H,
-                       G.cvec.p + l * H, G.agg.p + (size_t)l * n * H, G.pre.p + (size_t)l * n * H, hL(G, l + 1));
+    hipLaunchKernelGGL(kGnnMeanFold, dim3(1), dim3(kFinThreads), 0, s->stream, n, records, G.partials.p,
+                       P + G.lay.wg(l), P + G.lay.b(l), G.gmean.p + l * H, G.cvec.p + l * H);
+    auto layer = l + 1 < L ? kGnnLayerFwd<false> : kGnnLayerFwd<true>;
+    hipLaunchKernelGGL(layer, dim3(T.groups), dim3(256), 0, s->stream, n, T.n, T.per, (const __bf16 *)hL(G, l),
+                       s->dSliceOff.p, s->dSellCol.p, G.ahat.p, G.wT.p + (size_t)l * 128 * H, G.cvec.p + l * H,
+                       G.agg.p + (size_t)l * n * H, G.pre.p + (size_t)l * n * H, hL(G, l + 1), G.partials.p,
+                       P + G.lay.outW(), G.out.p);
+    records = T.groups;
   }
-  hipLaunchKernelGGL(kGnnOut, dim3(gridFor1(n)), dim3(256), 0, s->stream, n, (const __bf16 *)hL(G, L),
-                     P + G.lay.outW(), G.out.p);
   PH_CHECK(hipGetLastError());
 }
 
 // Loss of the last forward: against target t (error objective) or on the
 // residual r of the pair (residual objective, with the FP32 copy of A);
-// dout and dh_L for backward.
+// dout for backward.
 void gnnLoss(phase_hip_solver *s, const float *target, const float *r) {
   GnnState &G = *s->gnn;
-  const int n = s->rank;
+  const int n = s->rank, gr = gridFor1(n);
   if (s->learnedObjective == 1) {
     for (DBuf<float> *b : {&G.resC, &G.resQ, &G.resDq, &G.resG}) b->alloc(n);
     const int gs = std::max(1, (s->ord.nSlices + 3) / 4);
     hipLaunchKernelGGL(kGnnResC, dim3(g1(n)), dim3(256), 0, s->stream, n, G.out.p, G.sd.p, G.resC.p);
     hipLaunchKernelGGL((kSpmv<float>), dim3(gs), dim3(kRedBlock), 0, s->stream, n, s->ord.nSlices, s->dSliceOff.p,
                        s->dSellCol.p, s->dSell32.p, (const float *)G.resC.p, G.resQ.p);
-    hipLaunchKernelGGL(kGnnLossCos, dim3(gridFor1(n)), dim3(kRedBlock), 0, s->stream, n, G.resQ.p, r, G.scal.p,
-                       s->dPartials.p, s->dCounter.p);
+    hipLaunchKernelGGL(kGnnLossCos, dim3(gr), dim3(kRedBlock), 0, s->stream, n, G.resQ.p, r, s->dPartials.p);
+    hipLaunchKernelGGL(kGnnLossFinish, dim3(1), dim3(kFinBlock), 0, s->stream, s->dPartials.p, gr, G.scal.p);
     hipLaunchKernelGGL(kGnnResDq, dim3(g1(n)), dim3(256), 0, s->stream, n, G.resQ.p, r, G.scal.p, G.resDq.p);
     hipLaunchKernelGGL((kSpmv<float>), dim3(gs), dim3(kRedBlock), 0, s->stream, n, s->ord.nSlices, s->dSliceOff.p,
                        s->dSellCol.p, s->dSell32.p, (const float *)G.resDq.p, G.resG.p);
-    hipLaunchKernelGGL(kGnnResDout, dim3(g1((long)n * H)), dim3(256), 0, s->stream, n, G.resG.p, G.sd.p,
-                       G.params.p + G.lay.outW(), G.dOut.p, G.dh.p);
+    hipLaunchKernelGGL(kGnnResDout, dim3(g1(n)), dim3(256), 0, s->stream, n, G.resG.p, G.sd.p, G.dOut.p);
   } else {
-    hipLaunchKernelGGL(kGnnLossCos, dim3(gridFor1(n)), dim3(kRedBlock), 0, s->stream, n, G.out.p, target, G.scal.p,
-                       s->dPartials.p, s->dCounter.p);
-    hipLaunchKernelGGL(kGnnDout, dim3(g1((long)n * H)), dim3(256), 0, s->stream, n, G.out.p, target,
-                       G.params.p + G.lay.outW(), G.scal.p, G.dOut.p, G.dh.p);
+    hipLaunchKernelGGL(kGnnLossCos, dim3(gr), dim3(kRedBlock), 0, s->stream, n, G.out.p, target, s->dPartials.p);
+    hipLaunchKernelGGL(kGnnLossFinish, dim3(1), dim3(kFinBlock), 0, s->stream, s->dPartials.p, gr, G.scal.p);
+    hipLaunchKernelGGL(kGnnDout, dim3(g1(n)), dim3(256), 0, s->stream, n, G.out.p, target, G.scal.p, G.dOut.p);
   }
   PH_CHECK(hipGetLastError());
 }
@@ -713,29 +897,29 @@ void gnnBackward(phase_hip_solver *s) {
   GnnState &G = *s->gnn;
   const int n = s->rank, L = G.lay.L;
   const float *P = G.params.p;
-  const int nbO = std::min(1024, std::max(1, (n + 1023) / 1024));
+  const int nbO = std::min(kFwdGroups, std::max(1, (n + 31) / 32));
   hipLaunchKernelGGL(kGnnOutGrad, dim3(nbO), dim3(256), 0, s->stream, n, (const __bf16 *)hL(G, L), G.dOut.p,
                      G.partials.p);
-  hipLaunchKernelGGL(kSumPartials, dim3(1), dim3(128), 0, s->stream, nbO, H + 1, G.partials.p, G.grad.p + G.lay.outW());
-  const int nwg = (n + kWgRows - 1) / kWgRows;
-  const int nbW = (n + kChunkRows - 1) / kChunkRows;
+  hipLaunchKernelGGL(kSumPartials, dim3((H + 1 + H - 1) / H), dim3(kFinThreads), 0, s->stream, nbO, H + 1,
+                     G.partials.p, G.grad.p + G.lay.outW());
+  const Tiles T = tilesFor(n, kBwdGroups);
+  float *dagg[2] = {G.dagg.p, G.dagg.p + (size_t)n * H};
+  float *gterm = G.cvec.p;  // the forward's c vectors are no longer needed
   for (int l = L - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(kGnnBwdData, dim3(nwg), dim3(256), 0, s->stream, n, G.dh.p, G.pre.p + (size_t)l * n * H,
-                       G.wN.p + (size_t)l * 128 * H, G.dpre.p, G.dSA.p);
-    hipLaunchKernelGGL(kGnnBwdWeights, dim3(nbW), dim3(256), 0, s->stream, n, (const __bf16 *)hL(G, l),
-                       (const __bf16 *)(G.agg.p + (size_t)l * n * H), (const __bf16 *)G.dpre.p, G.partials.p);
-    // dWsm (128*64) and db (64) are contiguous in the partial record but
-    // separated by Wg in the parameter layout: sum in two pieces
-    hipLaunchKernelGGL(kSumPartialsStrided, dim3(g1(128 * H + H)), dim3(256), 0, s->stream, nbW, 128 * H + H,
-                       G.partials.p, G.grad.p + G.lay.wsm(l), 128 * H, G.grad.p + G.lay.b(l));
-    hipLaunchKernelGGL(kGnnGlobalGrad, dim3(1), dim3(64), 0, s->stream, n, G.gmean.p + l * H, G.grad.p + G.lay.b(l),
-                       P + G.lay.wg(l), G.grad.p + G.lay.wg(l), G.cvec.p + l * H);
-    hipLaunchKernelGGL((kGnnBwdCombine<float>), dim3(g1((long)n * H)), dim3(256), 0, s->stream, n, G.dh.p, G.dSA.p,
-                       s->dSliceOff.p, s->dSellCol.p, s->dSell32.p, G.sd.p, G.cvec.p + l * H);
+    auto layer = l == L - 1 ? kGnnLayerBwd<true> : kGnnLayerBwd<false>;
+    hipLaunchKernelGGL(layer, dim3(T.groups), dim3(256), 0, s->stream, n, T.n, T.per, G.dOut.p, P + G.lay.outW(),
+                       (const float *)G.dh.p, (const float *)dagg[(l + 1) & 1], (const float *)gterm, s->dSliceOff.p,
+                       s->dSellCol.p, G.ahat.p, G.pre.p + (size_t)l * n * H, (const __bf16 *)hL(G, l),
+                       (const __bf16 *)(G.agg.p + (size_t)l * n * H), G.wN.p + (size_t)l * 128 * H, G.dh.p,
+                       dagg[l & 1], G.partials.p);
+    hipLaunchKernelGGL(kGnnSumLayer, dim3(129), dim3(kFinThreads), 0, s->stream, n, T.groups, G.partials.p,
+                       G.gmean.p + l * H, P + G.lay.wg(l), G.grad.p + G.lay.wsm(l), G.grad.p + G.lay.b(l),
+                       G.grad.p + G.lay.wg(l), gterm);
   }
-  const int nbI = std::min(2048, std::max(1, (n + 255) / 256));
-  hipLaunchKernelGGL(kGnnInGrad, dim3(nbI), dim3(256), 0, s->stream, n, G.X.p, G.pre0.p, G.dh.p, G.partials.p);
-  hipLaunchKernelGGL(kSumPartials, dim3(g1((kGnnDin + 1) * H)), dim3(256), 0, s->stream, nbI, (kGnnDin + 1) * H,
+  const int nbI = std::min(kFwdGroups, std::max(1, (n + 15) / 16));
+  hipLaunchKernelGGL(kGnnInGrad, dim3(nbI), dim3(256), 0, s->stream, n, G.X.p, G.pre0.p, G.dh.p, dagg[0], gterm,
+                     s->dSliceOff.p, s->dSellCol.p, G.ahat.p, G.partials.p);
+  hipLaunchKernelGGL(kSumPartials, dim3(kGnnDin + 1), dim3(kFinThreads), 0, s->stream, nbI, (kGnnDin + 1) * H,
                      G.partials.p, G.grad.p + G.lay.inW());
   PH_CHECK(hipGetLastError());
 }
@@ -1008,7 +1192,7 @@ int phase_hip_learned_eval(phase_hip_solver *s, const double *r, const double *z
     const int n = s->rank;
     KrylovVecs<float> &K = s->k32;
     K.alloc(n);
-    DBuf<double> tmp;
+    DBuf<double> &tmp = G.stage;
     tmp.alloc(3 * (size_t)n);
     PH_CHECK(hipMemcpyAsync(tmp.p, r, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
     PH_CHECK(hipMemcpyAsync(tmp.p + n, z, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
@@ -1038,7 +1222,7 @@ int phase_hip_learned_apply(phase_hip_solver *s, const double *r, double *e) {
     PH_CHECK(hipSetDevice(s->device));
     gnnPrepare(s);
     const int n = s->rank;
-    DBuf<double> tmp;
+    DBuf<double> &tmp = s->gnn->stage;
     tmp.alloc(3 * (size_t)n);
     PH_CHECK(hipMemcpyAsync(tmp.p, r, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
     hipLaunchKernelGGL((kPermuteIn<double, double>), dim3(g1(n)), dim3(256), 0, s->stream, n, s->dPerm.p, tmp.p,

@@ -89,6 +89,40 @@ def test_forward_backward_match_fp64_oracle(hip, system, objective):
         assert rel(g[k], g_ref[k]) < 0.12, k
 
 
+@pytest.mark.parametrize("nx,ny", [(7, 9), (8, 8), (5, 13), (251, 251), (301, 300)])
+def test_layer_tiles_match_fp64_oracle(hip, oracle, nx, ny):
+    """Forward and backward at the edges of the 64-row tiles (63, 64 and 65
+    rows) and where a workgroup takes two tiles, in the backward kernel only
+    (63,001 rows) and in both (90,300 rows: the last workgroups' runs are
+    short).  The bounds are those of the test above: BF16 products of unit
+    round-off 2^-9 through six layers and back."""
+    from phase_amd import meshgen as G
+
+    m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, ny), sigma=0.5)
+    A = H.compact_sorted(rp, ci, v)
+    s = hip.HipSparseMatrixSolver(0, learnedObjective="error")
+    s.set(rp, ci, v)
+    rng = np.random.default_rng(nx)
+    p = NO.init_params(hidden=64, layers=6, seed=4)
+    for k in p:
+        if k.startswith("b"):
+            p[k] = rng.standard_normal(p[k].shape) * 0.05
+        p[k] = bf16_round(p[k])
+    s.learned_set_params(flatten(p).astype(np.float32))
+    Ah, sd, rowsum = NO.scaled_graph(A)
+    r = rng.standard_normal(len(b))
+    z = r / sd ** 2 * (1.0 + 0.3 * rng.standard_normal(len(b)))
+    X, sc = NO.features(r, z, sd, rowsum)
+    target = X[:, 0] + 0.5 * rng.standard_normal(len(b))
+    loss_ref, g_ref, out_ref = NO.loss_and_grad(Ah, X, p, target)
+    out, loss, grad = s.learned_eval(r, z, target)
+    assert rel(out, out_ref) < 3e-2
+    assert abs(loss - loss_ref) <= 5e-2 * loss_ref
+    assert rel(grad, flatten(g_ref)) < 0.12
+    again = s.learned_eval(r, z, target)
+    assert np.array_equal(out, again[0]) and loss == again[1] and np.array_equal(grad, again[2])
+
+
 def test_training_and_learned_mode(hip, system):
     rp, ci, v, b = system
     n = len(b)
