@@ -18,12 +18,16 @@ struct phase_hip_mesh {
   std::string err;
   int nNodes = 0, nCells = 0, nFaces = 0, nInterior = 0, nBoundary = 0;
   int maxDeg = 0;  // most interior links of one cell
+  bool repeated = false;  // a cell meets a neighbour (or itself) over more than one face
   std::vector<int> fNode1, fNode2, fL, fR;
   std::vector<int> iptr, iface, inb, bptr, bface;
   phase::DBuf<double> dXY, dVol, dCC, dFC, dSf;  // vectors interleaved (x, y)
   phase::DBuf<int> dCptr, dCind, dFNode1, dFNode2, dFL, dFR;
   phase::DBuf<int> dIptr, dIface, dInb, dBptr, dBface;
   phase::DBuf<double> dIDot, dIMs, dBDot, dBMs;  // per link: dot(r, Sf_out), |r|^2
+  phase::DBuf<int> dIfaceS, dBfaceS;  // per link: the face, kFlip set where Sf points into the cell
+  phase::DBuf<double> dFaceD, dFaceW;  // per face: r (interleaved), and the left cell's distance weight
+  phase::DBuf<double> dCourant;        // per cell: work space of the CICSAM weights
 };
 
 namespace phase {
@@ -31,6 +35,20 @@ namespace phase {
 struct Dv2 {
   double x, y;
 };
+
+// A vector of the interleaved fields as one 16-byte access (fields of callers
+// are only known to be 8-byte aligned, which the hardware takes).
+typedef double dv2_t __attribute__((ext_vector_type(2), aligned(8)));
+
+// Link entries of dIfaceS / dBfaceS: the outward test of Face::outwardNorm is a
+// property of the mesh, so the operators read its result with the face instead
+// of the face centroid (16 bytes a link less).
+constexpr int kFlip = (int)0x80000000;
+__device__ __forceinline__ int faceOf(int link) { return link & ~kFlip; }
+__device__ __forceinline__ Dv2 outwardOf(int link, const double *__restrict__ sf) {
+  const dv2_t n = *(const dv2_t *)(sf + 2 * (size_t)faceOf(link));
+  return link < 0 ? Dv2{-n.x, -n.y} : Dv2{n.x, n.y};
+}
 
 // Face::outwardNorm(point), Face.cpp:48-50: dot(centroid - point, normal) > 0
 // ? normal : -normal

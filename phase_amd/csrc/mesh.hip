@@ -103,13 +103,18 @@ __global__ void kLinkGeom(int nCells, const double *__restrict__ cc, const doubl
                           const int *__restrict__ iface, const int *__restrict__ inb,
                           const int *__restrict__ bptr, const int *__restrict__ bface,
                           double *__restrict__ idot, double *__restrict__ ims, double *__restrict__ bdot,
-                          double *__restrict__ bms) {
+                          double *__restrict__ bms, int *__restrict__ ifaceS, int *__restrict__ bfaceS) {
+  auto flip = [&](int f, Dv2 p) {  // outward()'s test
+    const double dx = fc[2 * f] - p.x, dy = fc[2 * f + 1] - p.y;
+    return (dx * sf[2 * f] + dy * sf[2 * f + 1]) > 0. ? f : f | kFlip;
+  };
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nCells; c += gridDim.x * blockDim.x) {
     const Dv2 p{cc[2 * c], cc[2 * c + 1]};
     for (int k = iptr[c]; k < iptr[c + 1]; ++k) {
       const int f = iface[k], nb = inb[k];
       const Dv2 s = outward(Dv2{fc[2 * f], fc[2 * f + 1]}, Dv2{sf[2 * f], sf[2 * f + 1]}, p);
       const double rx = cc[2 * nb] - p.x, ry = cc[2 * nb + 1] - p.y;
+      ifaceS[k] = flip(f, p);
       idot[k] = rx * s.x + ry * s.y;
       ims[k] = rx * rx + ry * ry;
     }
@@ -118,9 +123,33 @@ __global__ void kLinkGeom(int nCells, const double *__restrict__ cc, const doubl
       const Dv2 fcen{fc[2 * f], fc[2 * f + 1]};
       const Dv2 s = outward(fcen, Dv2{sf[2 * f], sf[2 * f + 1]}, p);
       const double rx = fcen.x - p.x, ry = fcen.y - p.y;
+      bfaceS[k] = flip(f, p);
       bdot[k] = rx * s.x + ry * s.y;
       bms[k] = rx * rx + ry * ry;
     }
+  }
+}
+
+// Per face: r = c_r - c_l (interior) or c_f - c_l (boundary), the vector of the
+// face gradients (ScalarGradient.cpp:34-52), and the left cell's interpolation
+// weight (Face::distanceWeight, Face.cpp:60-64; boundary 1).
+__global__ void kFaceLinks(int nFaces, const int *__restrict__ fl, const int *__restrict__ fr,
+                           const double *__restrict__ cc, const double *__restrict__ fc, double *__restrict__ d,
+                           double *__restrict__ w) {
+  for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nFaces; f += gridDim.x * blockDim.x) {
+    const int l = fl[f], r = fr[f];
+    if (r < 0) {
+      d[2 * f] = fc[2 * f] - cc[2 * l];
+      d[2 * f + 1] = fc[2 * f + 1] - cc[2 * l + 1];
+      w[f] = 1.;
+      continue;
+    }
+    d[2 * f] = cc[2 * r] - cc[2 * l];
+    d[2 * f + 1] = cc[2 * r + 1] - cc[2 * l + 1];
+    const double ax = fc[2 * f] - cc[2 * r], ay = fc[2 * f + 1] - cc[2 * r + 1];
+    const double bx = fc[2 * f] - cc[2 * l], by = fc[2 * f + 1] - cc[2 * l + 1];
+    const double l1 = sqrt(ax * ax + ay * ay), l2 = sqrt(bx * bx + by * by);
+    w[f] = l1 / (l1 + l2);
   }
 }
 
@@ -372,7 +401,12 @@ int phase_hip_mesh_create(phase_hip_mesh **out, int device, int nNodes, const do
     m->dFNode2.upload(m->fNode2, st);
     m->dFL.upload(m->fL, st);
     m->dFR.upload(m->fR, st);
-    for (int c = 0; c < nCells; ++c) m->maxDeg = std::max(m->maxDeg, m->iptr[c + 1] - m->iptr[c]);
+    for (int c = 0; c < nCells; ++c) {
+      m->maxDeg = std::max(m->maxDeg, m->iptr[c + 1] - m->iptr[c]);
+      for (int k = m->iptr[c]; k < m->iptr[c + 1]; ++k)
+        for (int j = m->iptr[c]; j <= k; ++j)
+          if (m->inb[k] == (j < k ? m->inb[j] : c)) m->repeated = true;
+    }
     m->dIptr.upload(m->iptr, st);
     m->dIface.upload(m->iface.empty() ? std::vector<int>{0} : m->iface, st);
     m->dInb.upload(m->inb.empty() ? std::vector<int>{0} : m->inb, st);
@@ -386,13 +420,20 @@ int phase_hip_mesh_create(phase_hip_mesh **out, int device, int nNodes, const do
     m->dIMs.alloc(std::max<size_t>(1, m->iface.size()));
     m->dBDot.alloc(std::max<size_t>(1, m->bface.size()));
     m->dBMs.alloc(std::max<size_t>(1, m->bface.size()));
+    m->dIfaceS.alloc(std::max<size_t>(1, m->iface.size()));
+    m->dBfaceS.alloc(std::max<size_t>(1, m->bface.size()));
+    m->dFaceD.alloc(2 * (size_t)m->nFaces);
+    m->dFaceW.alloc(m->nFaces);
+    m->dCourant.alloc(nCells);
     hipLaunchKernelGGL(kCellGeom, dim3(grid1(nCells)), dim3(256), 0, st, nCells, m->dCptr.p, m->dCind.p, m->dXY.p,
                        m->dVol.p, m->dCC.p);
     hipLaunchKernelGGL(kFaceGeom, dim3(grid1(m->nFaces)), dim3(256), 0, st, m->nFaces, m->dFNode1.p, m->dFNode2.p,
                        m->dXY.p, m->dFC.p, m->dSf.p);
     hipLaunchKernelGGL(kLinkGeom, dim3(grid1(nCells)), dim3(256), 0, st, nCells, m->dCC.p, m->dFC.p, m->dSf.p,
                        m->dIptr.p, m->dIface.p, m->dInb.p, m->dBptr.p, m->dBface.p, m->dIDot.p, m->dIMs.p,
-                       m->dBDot.p, m->dBMs.p);
+                       m->dBDot.p, m->dBMs.p, m->dIfaceS.p, m->dBfaceS.p);
+    hipLaunchKernelGGL(kFaceLinks, dim3(grid1(m->nFaces)), dim3(256), 0, st, m->nFaces, m->dFL.p, m->dFR.p,
+                       m->dCC.p, m->dFC.p, m->dFaceD.p, m->dFaceW.p);
     PH_CHECK(hipGetLastError());
     PH_CHECK(hipStreamSynchronize(st));
   });

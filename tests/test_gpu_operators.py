@@ -342,3 +342,51 @@ def test_copy_device(hip):
     c = hip.DeviceArray(np.zeros(3))
     with pytest.raises(hip.PhaseHipError):
         hip.DeviceArray(np.zeros(3)).copy_from(c)  # 24 bytes
+
+
+def _paired_columns(n):
+    """n columns of two pentagons that meet over two faces (a node between them
+    belongs to no other cell): a cell's neighbour comes up twice in its links."""
+    xy = [(x, y) for x in range(n + 1) for y in (0.0, 1.0, 2.0)] + [(x + 0.5, 1.25) for x in range(n)]
+    cind = []
+    for i in range(n):
+        a, b, m = 3 * i, 3 * (i + 1), 3 * (n + 1) + i
+        cind += [a, b, b + 1, m, a + 1, a + 1, m, b + 1, b + 2, a + 2]
+    return np.array(xy, float), 5 * np.arange(2 * n + 1, dtype=np.int32), np.array(cind, np.int32)
+
+
+@pytest.mark.parametrize("case", ["quad 255", "quad 256", "quad 257", "quad 1", "pairs 128", "pairs 129"])
+def test_row_blocks_match_oracle(hip, oracle, case):
+    """The row builder at the edges of its 256-row blocks, and on meshes where a
+    neighbour's column is touched twice: every operator and a merge of two, bit
+    for bit."""
+    kind, n = case.split()
+    n = int(n)
+    mesh = _paired_columns(n) if kind == "pairs" else H.rect_case(n, 1)
+    om, hm = oracle.Mesh(*mesh), hip.HipMesh(*mesh)
+    f = om.faces()
+    rng = np.random.default_rng(n)
+    bnd = np.flatnonzero(f["rcell"] < 0)
+    bc = np.full(om.n_faces, hip.BC_NORMAL_GRADIENT, np.int32)
+    bc[bnd] = rng.choice([hip.BC_FIXED, hip.BC_NORMAL_GRADIENT, hip.BC_SYMMETRY], len(bnd))
+    for ncomp in (1, 2):
+        fl = fields(om, 20 + ncomp)
+        key = "s" if ncomp == 1 else "v"
+        phiF, phi0C, phi0F = fl[key + "1f"], fl[key + "0c"], fl[key + "0f"]
+        d = dev(hip, u=fl["u"], u0=fl["u0"], bc=bc, phiF=phiF, phi0C=phi0C, phi0F=phi0F, g=fl["g"], g0=fl["g0"])
+        kw = dict(theta=0.5, bc_type=bc, phi_face=phiF, phi0_cell=phi0C, phi0_face=phi0F)
+        dkw = dict(theta=0.5, bc_type=d["bc"], phi_face=d["phiF"], phi0_cell=d["phi0C"], phi0_face=d["phi0F"])
+        od = oracle.div(om, fl["u"], fl["u0"], ncomp=ncomp, **kw)
+        hd = hip.HipEquation(hm, ncomp).div(d["u"], d["u0"], **dkw)
+        check_eq(hd, od)
+        check_eq(hip.HipEquation(hm, ncomp).divc(d["u"], d["u0"], **dkw),
+                 oracle.divc(om, fl["u"], fl["u0"], ncomp=ncomp, **kw))
+        check_eq(hip.HipEquation(hm, ncomp).ddt(0.5, d["phi0C"]), oracle.ddt(om, 0.5, phi0C, ncomp=ncomp))
+        for variant in range(4):
+            ol = oracle.laplacian(om, variant, ncomp=ncomp, gamma=0.75, gamma_face=fl["g"], gamma0_face=fl["g0"], **kw)
+            hl = hip.HipEquation(hm, ncomp).laplacian(variant, gamma=0.75, gamma_face=d["g"], gamma0_face=d["g0"],
+                                                      **dkw)
+            check_eq(hl, ol)
+            hl -= hd
+            ol -= od
+            check_eq(hl, ol)
