@@ -51,7 +51,7 @@ struct MlLevel {
   int nFiner = 0, nSlots = 0;
   // dense last level
   DBuf<int> cRowPtr, cColInd;
-  DBuf<double> cVals, dense, inv;
+  DBuf<double> cVals, dense, inv, invT;
   MlVecs<double> v64;
   MlVecs<float> v32;
   DBuf<MlScalars> msc;
@@ -833,6 +833,253 @@ __global__ __launch_bounds__(kRedBlock) void kMlJacDirection(int n, int nSlices,
   blockPartials<2>(d, partialsOut, blockIdx.x);
 }
 
+// ---------------------------------------------------------------- the last two levels
+// The coarse solve of the level above the dense one (Jacobi smoothing) in one
+// workgroup: the V cycle, or the K cycle's two flexible CG steps around it.
+// Such a level has a few hundred to a few thousand rows, and as launches of its
+// own every step of it costs a launch's latency (3 to 6 us) for well under a
+// microsecond of work.  Here a step costs a barrier: the rows' matrix entries
+// are read once, into registers (up to tailWidth a row, the rest from L2 at
+// every product), and the vector a product gathers from is in LDS.  Bound by
+// what one CU reads from L2: the matrix once and the dense inverse once per
+// cycle.  kMlTail keeps the arithmetic of the launches (each row's products in
+// slot order, the vectors rounded to T, sums in FP64) except for the order of
+// the restriction's and the dots' sums.
+// One K-cycle solve: 25.4 us for 2,500 rows (FP32 vectors, dense 175), 14.9 us for
+// 548 (FP64, dense 115), 12.0 us for 540 (FP32, dense 39); as nine launches 45, 45
+// and 36 us.  The V cycle over 276 rows 4.5 us (three launches: 13 us).
+constexpr int kTailBlock = 1024;
+constexpr int kTailRows = 4;  // rows per thread at most: 64 registers of matrix values
+// Entries of a row in registers: rows of brick aggregates have about 7, of graph
+// aggregates up to 14 and more.
+constexpr int tailWidth(int rows) { return rows == 1 ? 16 : rows == 2 ? 12 : 8; }
+template <class T>
+struct TailLevel {
+  int n, nd;
+  const int *sliceOff, *col;
+  const double *val;
+  const T *dinv;
+  const int *aggPtr, *pIdx;  // rows of each dense row, dense row of each row
+  const double *invT;        // inverse of the dense level, transposed, rows of 2 ceil(nd / 2)
+};
+
+template <class T, int R, bool KCYCLE>
+__global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *__restrict__ rIn,
+                                                      T *__restrict__ eOut, const Scalars *sc) {
+  if (sc->done) return;
+  constexpr int W = tailWidth(R);
+  __shared__ T xs[kTailBlock * R];                               // what the products gather from
+  __shared__ T z1s[KCYCLE ? kTailBlock * R : 1], q1s[KCYCLE ? kTailBlock * R : 1];
+  __shared__ T rc[kDenseMax], ec[kDenseMax];
+  __shared__ __align__(16) double part[2 * kTailBlock];
+  __shared__ double red[2][kTailBlock / 64];
+  __shared__ int ap[kDenseMax + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = L.n, nd = L.nd;
+  // matrix rows tid, tid + 1024, ..: a wavefront's rows are one SELL slice
+  double av[R][W];
+  unsigned ac[R][W / 2];  // columns, two to a register
+  int kw[R];                       // the slice's width, the same over the wavefront
+  int so[R], wide[R];              // entries past W: where, how many
+  T r[R], dinv[R];
+  int pi[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = tid + kTailBlock * i, slice = __builtin_amdgcn_readfirstlane(row >> 6);
+    const bool act = row < n;
+    so[i] = 0;
+    int K = 0;
+    if (64 * slice < n) {
+      so[i] = L.sliceOff[slice];
+      K = (L.sliceOff[slice + 1] - so[i]) >> 6;
+    }
+    wide[i] = act ? max(0, K - W) : 0;
+    kw[i] = __builtin_amdgcn_readfirstlane(K);
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      int c = -1;
+      double a = 0.;
+      if (q < K) {
+        c = L.col[so[i] + (q << 6) + lane];
+        a = L.val[so[i] + (q << 6) + lane];
+      }
+      // empty slots: 0 times the row's own entry
+      av[i][q] = c >= 0 ? a : 0.;
+      const unsigned u = (unsigned)(c >= 0 ? c : (act ? row : 0));
+      ac[i][q >> 1] = (q & 1) ? ac[i][q >> 1] | (u << 16) : u;
+    }
+    r[i] = act ? rIn[row] : (T)0;
+    dinv[i] = act ? L.dinv[row] : (T)0;
+    pi[i] = act ? L.pIdx[row] : 0;
+  }
+  for (int k = tid; k <= nd; k += kTailBlock) ap[k] = L.aggPtr[k];
+  // dense product: two rows a thread (16-byte loads), the columns in `segs` runs
+  const int pairs = (nd + 1) >> 1, segs = min(16, kTailBlock / pairs);
+  const int seg = tid / pairs, dk = tid - seg * pairs;
+  const int j0 = nd * seg / segs, j1 = nd * (seg + 1) / segs;
+
+  // A x for the thread's row i, x in xs
+  auto product = [&](int i) -> T {
+    double acc = 0.;
+#pragma unroll
+    for (int q0 = 0; q0 < W; q0 += 4)
+      if (q0 < kw[i]) {
+#pragma unroll
+        for (int q = q0; q < q0 + 4; ++q) {
+          const unsigned c = (q & 1) ? ac[i][q >> 1] >> 16 : ac[i][q >> 1] & 0xffffu;
+          acc = fma(av[i][q], (double)xs[c], acc);
+        }
+      }
+    for (int q = 0; q < wide[i]; ++q) {
+      const int idx = so[i] + ((W + q) << 6) + lane, c = L.col[idx];
+      if (c >= 0) acc = fma(L.val[idx], (double)xs[c], acc);
+    }
+    return (T)acc;
+  };
+  // block sums of two values, the same in every thread
+  auto sums = [&](double a, double b, double &sa, double &sb) {
+    a = waveSum(a);
+    b = waveSum(b);
+    if (lane == 0) {
+      red[0][wave] = a;
+      red[1][wave] = b;
+    }
+    __syncthreads();
+    sa = sb = 0.;
+#pragma unroll
+    for (int w = 0; w < kTailBlock / 64; ++w) {
+      sa += red[0][w];
+      sb += red[1][w];
+    }
+    __syncthreads();
+  };
+  // z = cycle applied to b (one entry per row of the thread): Jacobi, dense
+  // correction, Jacobi
+  auto cycle = [&](const T (&b)[R], T (&z)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      z[i] = dinv[i] * b[i];
+      xs[tid + kTailBlock * i] = z[i];
+    }
+    __syncthreads();
+    T t[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) t[i] = b[i] - product(i);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R; ++i) xs[tid + kTailBlock * i] = t[i];
+    __syncthreads();
+    for (int k0 = 0; k0 < nd; k0 += kTailBlock / 4) {  // four lanes per aggregate
+      const int k = k0 + (tid >> 2);
+      double d = 0.;
+      if (k < nd)
+        for (int i = ap[k] + (tid & 3); i < ap[k + 1]; i += 4) d += (double)xs[i];
+      d += __shfl_xor(d, 1, 64);
+      d += __shfl_xor(d, 2, 64);
+      if (k < nd && (tid & 3) == 0) rc[k] = (T)d;
+    }
+    __syncthreads();
+    if (seg < segs) {
+      const double2 *m = (const double2 *)L.invT + dk;
+      double ax = 0., ay = 0.;
+#pragma unroll 8
+      for (int j = j0; j < j1; ++j) {
+        const double2 v = m[(size_t)j * pairs];
+        const double x = (double)rc[j];
+        ax = fma(v.x, x, ax);
+        ay = fma(v.y, x, ay);
+      }
+      *(double2 *)&part[2 * tid] = double2{ax, ay};
+    }
+    __syncthreads();
+    if (tid < nd) {
+      double acc = 0.;
+      for (int q = 0; q < segs; ++q) acc += part[2 * pairs * q + tid];
+      ec[tid] = (T)acc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      z[i] = z[i] + ec[pi[i]];
+      xs[tid + kTailBlock * i] = z[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R; ++i) z[i] = z[i] + dinv[i] * (b[i] - product(i));
+    __syncthreads();  // xs is free
+  };
+
+  T z[R];
+  cycle(r, z);
+  if (!KCYCLE) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (tid + kTailBlock * i < n) eOut[tid + kTailBlock * i] = z[i];
+    return;
+  }
+  // first step: alpha1 = (z1, r) / (z1, A z1); r1 = r - alpha1 q1
+#pragma unroll
+  for (int i = 0; i < R; ++i) xs[tid + kTailBlock * i] = z[i];
+  __syncthreads();
+  double d0 = 0., d1 = 0., pq1, pr;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const T q = product(i);
+    const bool act = tid + kTailBlock * i < n;
+    z1s[tid + kTailBlock * i] = z[i];
+    q1s[tid + kTailBlock * i] = q;
+    if (act) {
+      d0 += (double)z[i] * (double)q;
+      d1 += (double)z[i] * (double)r[i];
+    }
+  }
+  sums(d0, d1, pq1, pr);
+  const T a1 = (T)((pq1 != 0. && isfinite(pq1) && isfinite(pr)) ? pr / pq1 : 0.);
+#pragma unroll
+  for (int i = 0; i < R; ++i) r[i] = r[i] - a1 * q1s[tid + kTailBlock * i];
+  // second step, its direction A-orthogonal to the first
+  cycle(r, z);
+  double zq, unused;
+  d0 = 0.;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    if (tid + kTailBlock * i < n) d0 += (double)z[i] * (double)q1s[tid + kTailBlock * i];
+  sums(d0, 0., zq, unused);
+  const T g = (T)((pq1 != 0. && isfinite(zq)) ? zq / pq1 : 0.);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    z[i] = z[i] - g * z1s[tid + kTailBlock * i];
+    xs[tid + kTailBlock * i] = z[i];
+  }
+  __syncthreads();
+  d0 = d1 = 0.;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const T q = product(i);
+    if (tid + kTailBlock * i < n) {
+      d0 += (double)z[i] * (double)q;
+      d1 += (double)z[i] * (double)r[i];
+    }
+  }
+  double pq2, pr2;
+  sums(d0, d1, pq2, pr2);
+  const T a2 = (T)((pq2 != 0. && isfinite(pq2) && isfinite(pr2)) ? pr2 / pq2 : 0.);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = tid + kTailBlock * i;
+    if (row < n) eOut[row] = a1 * z1s[row] + a2 * z[i];
+  }
+}
+
+// out = in^T (n x n), out's rows padded with a zero to an even length
+__global__ void kTransposeDense(int n, const double *__restrict__ in, double *__restrict__ out) {
+  const int pitch = (n + 1) & ~1;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n * pitch; t += gridDim.x * blockDim.x) {
+    const int j = t / pitch, k = t - j * pitch;
+    out[t] = k < n ? in[(size_t)k * n + j] : 0.;
+  }
+}
+
 // ---------------------------------------------------------------- host side
 phase_hip_solver *makeNested(phase_hip_solver *s) {
   auto *c = new phase_hip_solver();
@@ -854,6 +1101,32 @@ int elemGrid(long n) { return gridFor(n, 256, kElemCap); }
 template <class T>
 void cycle(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *r, T *e);
 
+// Level l and the dense level below it run as one workgroup (kMlTail): Jacobi
+// smoothing, and no more rows than its threads hold in registers.  A larger
+// level keeps its launches, whose blocks then share the work.
+bool tailLevel(const Multilevel &M, int l) {
+  const MlLevel &L = M.lv[l];
+  return L.sol && L.jacobi && L.n <= kTailBlock * kTailRows && !M.lv[l + 1].sol;
+}
+
+template <class T>
+void launchTail(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *r, T *e, bool kCycle) {
+  MlLevel &L = M.lv[l], &N = M.lv[l + 1];
+  phase_hip_solver *c = L.sol;
+  const TailLevel<T> t = {L.n,          N.n,          c->dSliceOff.p, c->dSellCol.p, c->dSell64.p,
+                          dinvOf<T>(L), N.finerAggPtr.p, N.pIdx.p,    N.invT.p};
+  auto go = [&](auto rows) {
+    constexpr int R = decltype(rows)::value;
+    auto kernel = kCycle ? kMlTail<T, R, true> : kMlTail<T, R, false>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kTailBlock), 0, s->stream, t, r, e, sc);
+  };
+  const int rows = (L.n + kTailBlock - 1) / kTailBlock;
+  if (rows <= 1) go(std::integral_constant<int, 1>());
+  else if (rows == 2) go(std::integral_constant<int, 2>());
+  else if (rows == 3) go(std::integral_constant<int, 3>());
+  else go(std::integral_constant<int, 4>());
+}
+
 // e = (approximate) A_l^-1 r at coarse level l
 template <class T>
 void coarseSolve(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *r, T *e) {
@@ -863,7 +1136,12 @@ void coarseSolve(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, c
     hipLaunchKernelGGL((kDenseApply<T>), dim3((L.n + 3) / 4), dim3(256), 0, st, L.n, L.inv.p, r, e, sc);
     return;
   }
-  if (!s->mlKCycle || l >= s->mlKLevels) {
+  const bool kCycle = s->mlKCycle && l < s->mlKLevels;
+  if (tailLevel(M, l)) {
+    launchTail<T>(s, M, l, sc, r, e, kCycle);
+    return;
+  }
+  if (!kCycle) {
     cycle<T>(s, M, l, sc, r, e);
     return;
   }
@@ -1103,6 +1381,7 @@ void mlEnsureHierarchy(phase_hip_solver *s) {
         L.cVals.alloc(std::max(1, L.nSlots));
         L.dense.alloc((size_t)c.n * c.n);
         L.inv.alloc((size_t)c.n * c.n);
+        L.invT.alloc((size_t)c.n * (c.n + 1));
         for (int i = 0; i < nFiner; ++i) pIdx[i] = c.aggOfRow[i];
       } else {
         L.restRow.upload(L.sol->ord.perm, st);
@@ -1151,6 +1430,7 @@ void mlEnsureValues(phase_hip_solver *s, bool single) {
         hipLaunchKernelGGL(kDenseFill, dim3(elemGrid(L.n)), dim3(256), 0, st, L.n, L.cRowPtr.p, L.cColInd.p,
                            L.cVals.p, L.dense.p);
         denseInverse(st, L.n, L.dense.p, L.inv.p, s->dErr.p, s->mlDensePivot != 0);
+        hipLaunchKernelGGL(kTransposeDense, dim3(elemGrid((long)L.n * L.n)), dim3(256), 0, st, L.n, L.inv.p, L.invT.p);
         int e = 0;
         PH_CHECK(hipMemcpyAsync(&e, s->dErr.p, sizeof(int), hipMemcpyDeviceToHost, st));
         PH_CHECK(hipStreamSynchronize(st));

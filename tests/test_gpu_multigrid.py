@@ -175,3 +175,33 @@ def test_multigrid_graph_aggregates_wide_coarse_rows(hip, oracle):
         assert np.linalg.norm(b - A @ x) <= 1.5e-8 * np.linalg.norm(b)
         assert len(s.multigrid_levels()) >= 4
         assert s.n_iters() <= 150, s.n_iters()
+
+
+@pytest.mark.parametrize("cycle", ["K", "V"])
+@pytest.mark.parametrize("nx,rows", [(128, 1), (170, 1), (180, 2), (250, 3), (350, 4), (360, 5)])
+def test_last_levels_match_direct(hip, oracle, nx, rows, cycle):
+    """The level above the dense one in one workgroup, at 1 to 4 rows per thread
+    (565 to 4,084 rows, 979 and 1,100 and 4,084 at the edges; graph aggregates,
+    whose rows are partly wider than the entries held in registers), and as
+    launches above that (4,316 rows).  A solve to 1e-10 is within
+    cond(A) 1e-10 of the direct one; cond(A) is below 16 nx^2 for these
+    coefficients (8 / pi^2 nx^2 times the spread e^(4 sigma) within four
+    deviations, sigma = 0.5).  A wrong coarse correction shows in the iteration
+    count: K cycles take 38 to 42, V cycles twice that."""
+    m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, nx), sigma=0.5)
+    A = H.compact_sorted(rp, ci, v)
+    x_ref = spla.splu(A.tocsc()).solve(b)
+    for mode in ("fp64", "mixed"):
+        s = hip.HipSparseMatrixSolver(0, tolerance=1e-10, maxIters=2000, solver="cg", mode=mode,
+                                      preconditioner="multigrid", multigridDenseRows=512, multigridCycle=cycle)
+        s.set(rp, ci, v)
+        s.set_rhs(b)
+        s.solve()
+        x = s.x()
+        lv = s.multigrid_levels()
+        assert (lv[-2] + 1023) // 1024 == rows, lv
+        assert np.linalg.norm(x - x_ref) <= 16 * nx * nx * 1e-10 * np.linalg.norm(x_ref)
+        assert s.n_iters() <= (60 if cycle == "K" else 130)
+        s.zero_guess()
+        s.solve()
+        assert np.array_equal(s.x(), x)
