@@ -43,6 +43,9 @@ struct MlLevel {
   bool jacobi = false;              // damped Jacobi smoothing (dinv) instead of the ILU(0) factor
   DBuf<double> dinv64;              // omega / a_ii in solver order
   DBuf<float> dinv32;
+  int blockWidth = 0;               // ILU(0) level that can run as kMlTail: its longest block (0: cannot)
+  DBuf<double> binv64;              // its blocks' inverses
+  DBuf<float> binv32;
   // maps from the finer level
   DBuf<int> galPtr, galSrc;         // coarse slot q = sum of finer caller slots galSrc[galPtr[q] ..]
   DBuf<int> restRow;                // this level's solver row -> aggregate of the finer level (dense: identity)
@@ -98,6 +101,16 @@ const double *dinvOf<double>(const MlLevel &L) {
 template <>
 const float *dinvOf<float>(const MlLevel &L) {
   return L.dinv32.p;
+}
+template <class T>
+const T *binvOf(const MlLevel &L);
+template <>
+const double *binvOf<double>(const MlLevel &L) {
+  return L.binv64.p;
+}
+template <>
+const float *binvOf<float>(const MlLevel &L) {
+  return L.binv32.p;
 }
 // the ILU(0) factor a level applies in precision T
 template <class T>
@@ -834,8 +847,11 @@ __global__ __launch_bounds__(kRedBlock) void kMlJacDirection(int n, int nSlices,
 }
 
 // ---------------------------------------------------------------- the last two levels
-// The coarse solve of the level above the dense one (Jacobi smoothing) in one
-// workgroup: the V cycle, or the K cycle's two flexible CG steps around it.
+// The coarse solve of the level above the dense one in one workgroup: the V
+// cycle, or the K cycle's two flexible CG steps around it, smoothed by damped
+// Jacobi or by the block-diagonal ILU(0), whose blocks are the aggregates and
+// are applied as explicit inverses (kBlockInverse; a block's level-by-level
+// sweeps would cost a barrier a level).
 // Such a level has a few hundred to a few thousand rows, and as launches of its
 // own every step of it costs a launch's latency (3 to 6 us) for well under a
 // microsecond of work.  Here a step costs a barrier: the rows' matrix entries
@@ -847,8 +863,11 @@ __global__ __launch_bounds__(kRedBlock) void kMlJacDirection(int n, int nSlices,
 // the restriction's and the dots' sums.
 // One K-cycle solve: 25.4 us for 2,500 rows (FP32 vectors, dense 175), 14.9 us for
 // 548 (FP64, dense 115), 12.0 us for 540 (FP32, dense 39); as nine launches 45, 45
-// and 36 us.  The V cycle over 276 rows 4.5 us (three launches: 13 us).
+// and 36 us.  The V cycle over 276 rows 4.5 us (three launches: 13 us).  With
+// ILU(0) smoothing 412 rows take 15.6 us a K cycle (FP32; sixteen launches 64 us)
+// and 540 rows 8.9 us a V cycle (FP64; five launches 21 us).
 constexpr int kTailBlock = 1024;
+constexpr int kTailInvBytes = 104 * 1024;  // LDS for block inverses, beside at most 52 KB of vectors
 constexpr int kTailRows = 4;  // rows per thread at most: 64 registers of matrix values
 // Entries of a row in registers: rows of brick aggregates have about 7, of graph
 // aggregates up to 14 and more.
@@ -858,12 +877,14 @@ struct TailLevel {
   int n, nd;
   const int *sliceOff, *col;
   const double *val;
-  const T *dinv;
+  const T *dinv;             // Jacobi: omega / a_ii
+  const T *binv;             // ILU: entry e of row i of its block's inverse at e n + i
+  int blockWidth;            // ILU: rows of the longest block
   const int *aggPtr, *pIdx;  // rows of each dense row, dense row of each row
   const double *invT;        // inverse of the dense level, transposed, rows of 2 ceil(nd / 2)
 };
 
-template <class T, int R, bool KCYCLE>
+template <class T, int R, bool KCYCLE, bool ILU>
 __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *__restrict__ rIn,
                                                       T *__restrict__ eOut, const Scalars *sc) {
   if (sc->done) return;
@@ -874,8 +895,17 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
   __shared__ __align__(16) double part[2 * kTailBlock];
   __shared__ double red[2][kTailBlock / 64];
   __shared__ int ap[kDenseMax + 1];
+  // the block inverses, where they fit (one row a thread): a K cycle applies
+  // them four times, and out of L2 each costs three round trips
+  constexpr int kInvLds = ILU && R == 1 ? kTailInvBytes / (int)sizeof(T) : 1;
+  __shared__ T bl[kInvLds];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = L.n, nd = L.nd;
+  const bool invLds = ILU && R == 1 && n * L.blockWidth <= kInvLds;
+  if (invLds) {
+#pragma unroll 8
+    for (int q = tid; q < n * L.blockWidth; q += kTailBlock) bl[q] = L.binv[q];
+  }
   // matrix rows tid, tid + 1024, ..: a wavefront's rows are one SELL slice
   double av[R][W];
   unsigned ac[R][W / 2];  // columns, two to a register
@@ -909,10 +939,11 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
       ac[i][q >> 1] = (q & 1) ? ac[i][q >> 1] | (u << 16) : u;
     }
     r[i] = act ? rIn[row] : (T)0;
-    dinv[i] = act ? L.dinv[row] : (T)0;
+    dinv[i] = act && !ILU ? L.dinv[row] : (T)0;
     pi[i] = act ? L.pIdx[row] : 0;
   }
   for (int k = tid; k <= nd; k += kTailBlock) ap[k] = L.aggPtr[k];
+  if (ILU) __syncthreads();  // the first smoothing reads them
   // dense product: two rows a thread (16-byte loads), the columns in `segs` runs
   const int pairs = (nd + 1) >> 1, segs = min(16, kTailBlock / pairs);
   const int seg = tid / pairs, dk = tid - seg * pairs;
@@ -953,14 +984,41 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
     }
     __syncthreads();
   };
-  // z = cycle applied to b (one entry per row of the thread): Jacobi, dense
-  // correction, Jacobi
-  auto cycle = [&](const T (&b)[R], T (&z)[R]) {
+  // s = M^-1 b of the smoother (xs free before and after)
+  auto smooth = [&](const T (&b)[R], T (&s)[R]) {
+    if (!ILU) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) s[i] = dinv[i] * b[i];
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) xs[tid + kTailBlock * i] = b[i];
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      z[i] = dinv[i] * b[i];
-      xs[tid + kTailBlock * i] = z[i];
+      const int row = tid + kTailBlock * i;
+      T acc = 0;
+      if (row < n) {
+        const int c0 = ap[pi[i]], m = ap[pi[i] + 1] - c0;
+        if (invLds) {
+#pragma unroll 4
+          for (int e = 0; e < m; ++e) acc = fma(bl[e * n + row], xs[c0 + e], acc);
+        } else {
+          const T *a = L.binv + row;
+#pragma unroll 8
+          for (int e = 0; e < m; ++e) acc = fma(a[(size_t)e * n], xs[c0 + e], acc);
+        }
+      }
+      s[i] = acc;
     }
+    __syncthreads();
+  };
+  // z = cycle applied to b (one entry per row of the thread): smoothing, dense
+  // correction, smoothing
+  auto cycle = [&](const T (&b)[R], T (&z)[R]) {
+    smooth(b, z);
+#pragma unroll
+    for (int i = 0; i < R; ++i) xs[tid + kTailBlock * i] = z[i];
     __syncthreads();
     T t[R];
 #pragma unroll
@@ -1005,8 +1063,12 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < R; ++i) z[i] = z[i] + dinv[i] * (b[i] - product(i));
+    for (int i = 0; i < R; ++i) t[i] = b[i] - product(i);
     __syncthreads();  // xs is free
+    T s[R];
+    smooth(t, s);
+#pragma unroll
+    for (int i = 0; i < R; ++i) z[i] = z[i] + s[i];
   };
 
   T z[R];
@@ -1071,6 +1133,36 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
   }
 }
 
+// Explicit inverses of the ILU(0) blocks of a block-diagonal factor, one
+// wavefront per block (at most 64 rows), lane j solving for unit vector j: entry e
+// of row i of its block's inverse at inv[e n + i].
+__global__ __launch_bounds__(64) void kBlockInverse(IluDev<double> L, double *__restrict__ inv) {
+  __shared__ double x[64][64];
+  const int b = blockIdx.x, j = threadIdx.x;
+  const BlockInfo B = L.blocks[b];
+  const double *facU = L.fac + L.nLSlots;
+  for (int i = 0; i < B.nRows; ++i) {
+    const unsigned info = L.lanes[(size_t)b * 64 + i].info;
+    double a = i == j ? 1. : 0.;
+    for (int e = 0; e < (int)(info & 15u); ++e) {
+      const int s = B.lOff + (e << 6) + i;
+      a = fma(-L.fac[s], x[L.lCol[s] - B.rowStart][j], a);
+    }
+    x[i][j] = a;
+  }
+  for (int i = B.nRows - 1; i >= 0; --i) {
+    const unsigned info = L.lanes[(size_t)b * 64 + i].info;
+    double a = x[i][j];
+    for (int e = 0; e < (int)((info >> 10) & 15u); ++e) {
+      const int s = B.uOff + (e << 6) + i;
+      a = fma(-facU[s], x[L.uCol[s] - B.rowStart][j], a);
+    }
+    a *= L.fac[L.nLSlots + L.nUSlots + L.n + B.rowStart + i];
+    x[i][j] = a;
+    if (j < B.nRows) inv[(size_t)j * L.n + B.rowStart + i] = a;
+  }
+}
+
 // out = in^T (n x n), out's rows padded with a zero to an even length
 __global__ void kTransposeDense(int n, const double *__restrict__ in, double *__restrict__ out) {
   const int pitch = (n + 1) & ~1;
@@ -1101,12 +1193,16 @@ int elemGrid(long n) { return gridFor(n, 256, kElemCap); }
 template <class T>
 void cycle(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *r, T *e);
 
-// Level l and the dense level below it run as one workgroup (kMlTail): Jacobi
-// smoothing, and no more rows than its threads hold in registers.  A larger
-// level keeps its launches, whose blocks then share the work.
+// Level l and the dense level below it run as one workgroup (kMlTail): no more
+// rows than its threads hold in registers, and with ILU(0) smoothing
+// block-diagonal in the aggregates and at most kTailIluRows, whose block
+// inverses (some 20 entries a row) are read from L2 at every smoothing.  A
+// larger level keeps its launches, whose blocks then share the work.
+constexpr int kTailIluRows = 2 * kTailBlock;
 bool tailLevel(const Multilevel &M, int l) {
   const MlLevel &L = M.lv[l];
-  return L.sol && L.jacobi && L.n <= kTailBlock * kTailRows && !M.lv[l + 1].sol;
+  if (!L.sol || M.lv[l + 1].sol) return false;
+  return L.jacobi ? L.n <= kTailBlock * kTailRows : L.blockWidth > 0;
 }
 
 template <class T>
@@ -1114,13 +1210,23 @@ void launchTail(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, co
   MlLevel &L = M.lv[l], &N = M.lv[l + 1];
   phase_hip_solver *c = L.sol;
   const TailLevel<T> t = {L.n,          N.n,          c->dSliceOff.p, c->dSellCol.p, c->dSell64.p,
-                          dinvOf<T>(L), N.finerAggPtr.p, N.pIdx.p,    N.invT.p};
+                          dinvOf<T>(L), binvOf<T>(L), L.blockWidth,    N.finerAggPtr.p, N.pIdx.p, N.invT.p};
   auto go = [&](auto rows) {
     constexpr int R = decltype(rows)::value;
-    auto kernel = kCycle ? kMlTail<T, R, true> : kMlTail<T, R, false>;
+    auto kernel = kCycle ? kMlTail<T, R, true, false> : kMlTail<T, R, false, false>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kTailBlock), 0, s->stream, t, r, e, sc);
+  };
+  auto goIlu = [&](auto rows) {
+    constexpr int R = decltype(rows)::value;
+    auto kernel = kCycle ? kMlTail<T, R, true, true> : kMlTail<T, R, false, true>;
     hipLaunchKernelGGL(kernel, dim3(1), dim3(kTailBlock), 0, s->stream, t, r, e, sc);
   };
   const int rows = (L.n + kTailBlock - 1) / kTailBlock;
+  if (!L.jacobi) {
+    if (rows <= 1) goIlu(std::integral_constant<int, 1>());
+    else goIlu(std::integral_constant<int, 2>());
+    return;
+  }
   if (rows <= 1) go(std::integral_constant<int, 1>());
   else if (rows == 2) go(std::integral_constant<int, 2>());
   else if (rows == 3) go(std::integral_constant<int, 3>());
@@ -1383,6 +1489,22 @@ void mlEnsureHierarchy(phase_hip_solver *s) {
         L.inv.alloc((size_t)c.n * c.n);
         L.invT.alloc((size_t)c.n * (c.n + 1));
         for (int i = 0; i < nFiner; ++i) pIdx[i] = c.aggOfRow[i];
+        // can the ILU(0) level above run as kMlTail: its blocks are the aggregates
+        if (level > 0) {
+          MlLevel &U = M->lv[level - 1];
+          if (!U.jacobi && U.sol->blockJacobi && U.n <= kTailIluRows && (int)fine->blocks.size() == c.n) {
+            int width = 0;
+            for (int a = 0; a < c.n; ++a) {
+              const BlockInfo &B = fine->blocks[a];
+              if (B.rowStart != fine->aggPtr[a] || B.nRows != fine->aggPtr[a + 1] - fine->aggPtr[a]) {
+                width = 0;
+                break;
+              }
+              width = std::max(width, B.nRows);
+            }
+            U.blockWidth = width;
+          }
+        }
       } else {
         L.restRow.upload(L.sol->ord.perm, st);
         for (int i = 0; i < nFiner; ++i) pIdx[i] = L.sol->ord.iperm[c.aggOfRow[i]];
@@ -1422,6 +1544,11 @@ void mlEnsureValues(phase_hip_solver *s, bool single) {
                              L.sol->dSellCol.p, L.sol->dSell64.p, s->mlJacobiWeight, L.dinv64.p);
         } else {
           ensureFactor64(L.sol);
+          if (L.blockWidth > 0) {
+            L.binv64.alloc((size_t)L.blockWidth * L.n);
+            hipLaunchKernelGGL(kBlockInverse, dim3(L.sol->ord.nBlocks), dim3(64), 0, st,
+                               iluDev<double>(L.sol, L.sol->dFac64.p), L.binv64.p);
+          }
         }
         finer = L.sol->dVals.p;
       } else {
@@ -1459,6 +1586,12 @@ void mlEnsureValues(phase_hip_solver *s, bool single) {
                              L.dinv32.p);
         } else if (L.sol) {
           ensureSingle(L.sol);
+          if (L.blockWidth > 0) {
+            const int m = (int)L.binv64.n;
+            L.binv32.alloc(m);
+            hipLaunchKernelGGL((kConvert<double, float>), dim3(elemGrid(m)), dim3(256), 0, st, m, L.binv64.p,
+                               L.binv32.p);
+          }
         }
       M.singleValid = true;
     }

@@ -205,3 +205,28 @@ def test_last_levels_match_direct(hip, oracle, nx, rows, cycle):
         s.zero_guess()
         s.solve()
         assert np.array_equal(s.x(), x)
+
+
+@pytest.mark.parametrize("solver", ["bicgstab", "gmres"])
+@pytest.mark.parametrize("nx,rows", [(128, 1), (170, 1), (180, 2), (250, 3)])
+def test_last_levels_ilu_match_direct(hip, oracle, nx, rows, solver):
+    """As above with ILU(0)-smoothed coarse levels: V cycles under BiCGStab, K
+    cycles under GMRES; 565 to 1,100 rows in one workgroup (block inverses),
+    2,110 as launches."""
+    m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, nx), sigma=0.5)
+    A = H.compact_sorted(rp, ci, v)
+    x_ref = spla.splu(A.tocsc()).solve(b)
+    for mode in ("fp64", "mixed"):
+        s = hip.HipSparseMatrixSolver(0, tolerance=1e-10, maxIters=2000, solver=solver, mode=mode,
+                                      preconditioner="multigrid")
+        s.set(rp, ci, v)
+        s.set_rhs(b)
+        s.solve()
+        x = s.x()
+        lv = s.multigrid_levels()
+        assert (lv[1] + 1023) // 1024 == rows, lv
+        assert np.linalg.norm(x - x_ref) <= 16 * nx * nx * 1e-10 * np.linalg.norm(x_ref)
+        assert s.n_iters() <= 200
+        s.zero_guess()
+        s.solve()
+        assert np.array_equal(s.x(), x)
