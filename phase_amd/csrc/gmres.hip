@@ -50,6 +50,12 @@ constexpr int kGmGroup = 8;
 constexpr double kGmMixedDrop = 1e-5;  // a mixed cycle's reduction of the residual estimate
 constexpr int kGmMixedStall = 3;
 
+// Blocks of the dot products, at most: one per CU.  A block's sums of kGmGroup
+// vectors cost it as much as several rows a thread, and every kGmAxpy block
+// reads the partials (at 200,000 rows one row a thread, 782 blocks, took
+// 13.2 us); up to 65,536 rows a row a thread keeps more CUs busy.
+constexpr int kGmDotBlocks = 256;
+
 // partials of (w, V_j) for the kGmGroup vectors j = 8 blockIdx.y + q < k
 template <class T>
 __global__ __launch_bounds__(kRedBlock) void kGmDots(int n, int k, const T *__restrict__ V,
@@ -69,36 +75,36 @@ __global__ __launch_bounds__(kRedBlock) void kGmDots(int n, int k, const T *__re
   blockPartials<kGmGroup>(d, partials + (size_t)g0 * gridDim.x, blockIdx.x);
 }
 
-// h_j = sum of the G partials of vector j (one wavefront per j, fixed order);
-// the Hessenberg column takes h (first pass) or adds it (second pass)
-__global__ __launch_bounds__(kFinBlock) void kGmDotsFinish(int k, int G, const double *partials, double *hcur,
-                                                           double *Hcol, int accumulate, const Scalars *sc) {
-  if (sc->done) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int j = wave; j < k; j += kFinBlock / 64) {
-    double acc = 0.;
-    for (int b = lane; b < G; b += 64) acc += partials[(size_t)j * G + b];
-    acc = waveSum(acc);
-    if (lane == 0) {
-      hcur[j] = acc;
-      Hcol[j] = accumulate ? Hcol[j] + acc : acc;
-    }
-  }
-}
-
 // w -= sum_{j<k} h_j V_j (in FP64, stored in T); with NORM the partials of
-// (w, w) of the stored w
+// (w, w) of the stored w.  h_j is the sum of vector j's G partials, formed by
+// every block in the same fixed order (7.0 us at 200,000 rows and 16 vectors;
+// 4.3 us with a finisher of one block in between that took 6.9 us); block 0 sets the Hessenberg column to it
+// (first pass) or adds it (second pass).
 template <class T, bool NORM>
-__global__ __launch_bounds__(kRedBlock) void kGmAxpy(int n, int k, const T *__restrict__ V,
-                                                     const double *__restrict__ hcur, T *__restrict__ w,
-                                                     double *partials, const Scalars *sc) {
+__global__ __launch_bounds__(kRedBlock) void kGmAxpy(int n, int k, const T *__restrict__ V, int G,
+                                                     const double *__restrict__ dotPart, double *Hcol,
+                                                     T *__restrict__ w, double *partials, const Scalars *sc) {
   if (sc->done) return;
   __shared__ double h[kGmMaxRestart + 1];
-  for (int j = threadIdx.x; j < k; j += kRedBlock) h[j] = hcur[j];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int j = wave; j < k; j += kRedBlock / 64) {
+    double t[kGmDotBlocks / 64], acc = 0.;
+#pragma unroll
+    for (int u = 0; u < kGmDotBlocks / 64; ++u)
+      t[u] = lane + 64 * u < G ? dotPart[(size_t)j * G + lane + 64 * u] : 0.;
+#pragma unroll
+    for (int u = 0; u < kGmDotBlocks / 64; ++u) acc += t[u];
+    acc = waveSum(acc);
+    if (lane == 0) {
+      h[j] = acc;
+      if (blockIdx.x == 0) Hcol[j] = NORM ? Hcol[j] + acc : acc;
+    }
+  }
   __syncthreads();
   double d[1] = {0.};
   for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
     double v = (double)w[i];
+#pragma unroll 8
     for (int j = 0; j < k; ++j) v = fma(-h[j], (double)V[(size_t)j * n + i], v);
     const T vt = (T)v;
     w[i] = vt;
@@ -113,17 +119,26 @@ __global__ __launch_bounds__(kFinBlock) void kGmGivens(int j, int ld, const doub
                                                        double *cs, double *sn, double *g, double *vscale,
                                                        Scalars *sc) {
   if (sc->done) return;
+  // the column and the rotations come in together: read one by one in the
+  // chain below they cost a round trip each (6.7 us; 3.4 us so)
+  __shared__ double sh[kGmMaxRestart + 1], scs[kGmMaxRestart], ssn[kGmMaxRestart];
+  double *h = H + (size_t)j * ld;
+  if ((int)threadIdx.x <= j) sh[threadIdx.x] = h[threadIdx.x];
+  if ((int)threadIdx.x < j) {
+    scs[threadIdx.x] = cs[threadIdx.x];
+    ssn[threadIdx.x] = sn[threadIdx.x];
+  }
   double d[1];
   finishPartials<1, kFinBlock>(partials, G, d);
   if (threadIdx.x != 0) return;
-  double *h = H + (size_t)j * ld;
   const double hn = sqrt(d[0]);
+  double top = sh[0];
   for (int i = 0; i < j; ++i) {
-    const double a = h[i], b = h[i + 1];
-    h[i] = cs[i] * a + sn[i] * b;
-    h[i + 1] = -sn[i] * a + cs[i] * b;
+    const double a = top, b = sh[i + 1];
+    h[i] = scs[i] * a + ssn[i] * b;
+    top = -ssn[i] * a + scs[i] * b;
   }
-  const double a = h[j], b = hn;
+  const double a = top, b = hn;
   const double r = hypot(a, b);
   const double c = r > 0. ? a / r : 1., s = r > 0. ? b / r : 0.;
   cs[j] = c;
@@ -247,20 +262,21 @@ int gmresCycles(phase_hip_solver *s, double b2, int budget, bool *stalled) {
   hipStream_t st = s->stream;
   const IluDev<T> L = iluDev<T>(s, factor<T>(s));
   const int G = gridFor(n, kRedBlock, kRedCap);
+  const int Gd = gridFor(n, kRedBlock, kGmDotBlocks), Ga = gridFor(n, kRedBlock, 2 * kGmDotBlocks);
   const int groups = (m + 1 + kGmGroup - 1) / kGmGroup;
   gmBasis<T>(s).alloc((size_t)(m + 1) * n);
   gmPrec<T>(s).alloc((size_t)m * n);
   s->gmH.alloc((size_t)ld * m);
-  // small: cs (m), sn (m), g (m + 1), y (m), hcur (m + 1), vscale (1)
-  s->gmSmall.alloc((size_t)5 * (m + 1) + 1);
-  s->gmPart.alloc((size_t)groups * kGmGroup * G + G);
+  // small: cs (m), sn (m), g (m + 1), y (m), vscale (1)
+  s->gmSmall.alloc((size_t)4 * (m + 1) + 1);
+  s->gmPart.alloc((size_t)groups * kGmGroup * Gd + Ga);
   krylov<T>(s).alloc(n);
   s->dR64.alloc(n);
   T *V = gmBasis<T>(s).p, *Z = gmPrec<T>(s).p;
   double *H = s->gmH.p;
-  double *cs = s->gmSmall.p, *sn = cs + (m + 1), *g = sn + (m + 1), *y = g + (m + 1), *hcur = y + (m + 1);
-  double *vscale = hcur + (m + 1);
-  double *dotPart = s->gmPart.p, *normPart = dotPart + (size_t)groups * kGmGroup * G;
+  double *cs = s->gmSmall.p, *sn = cs + (m + 1), *g = sn + (m + 1), *y = g + (m + 1);
+  double *vscale = y + (m + 1);
+  double *dotPart = s->gmPart.p, *normPart = dotPart + (size_t)groups * kGmGroup * Gd;
   Scalars *sc = s->dSc.p;
   const double tol2 = s->tol * s->tol * b2;
   const int ge = gridFor(n, 256, kElemCap);
@@ -312,18 +328,13 @@ int gmresCycles(phase_hip_solver *s, double b2, int budget, bool *stalled) {
         hipLaunchKernelGGL((kSpmv<T, double>), dim3(spmvGrid(s)), dim3(kRedBlock), 0, st, n, s->ord.nSlices,
                            s->dSliceOff.p, s->dSellCol.p, s->dSell64.p, (const T *)zj, w);
         for (int pass = 0; pass < 2; ++pass) {
-          hipLaunchKernelGGL((kGmDots<T>), dim3(G, (j + 1 + kGmGroup - 1) / kGmGroup), dim3(kRedBlock), 0, st, n,
+          hipLaunchKernelGGL((kGmDots<T>), dim3(Gd, (j + 1 + kGmGroup - 1) / kGmGroup), dim3(kRedBlock), 0, st, n,
                              j + 1, (const T *)V, (const T *)w, dotPart, (const Scalars *)sc);
-          hipLaunchKernelGGL(kGmDotsFinish, dim3(1), dim3(kFinBlock), 0, st, j + 1, G, (const double *)dotPart,
-                             hcur, H + (size_t)j * ld, pass, (const Scalars *)sc);
-          if (pass == 0)
-            hipLaunchKernelGGL((kGmAxpy<T, false>), dim3(G), dim3(kRedBlock), 0, st, n, j + 1, (const T *)V,
-                               (const double *)hcur, w, normPart, (const Scalars *)sc);
-          else
-            hipLaunchKernelGGL((kGmAxpy<T, true>), dim3(G), dim3(kRedBlock), 0, st, n, j + 1, (const T *)V,
-                               (const double *)hcur, w, normPart, (const Scalars *)sc);
+          auto axpy = pass == 0 ? kGmAxpy<T, false> : kGmAxpy<T, true>;
+          hipLaunchKernelGGL(axpy, dim3(Ga), dim3(kRedBlock), 0, st, n, j + 1, (const T *)V, Gd,
+                             (const double *)dotPart, H + (size_t)j * ld, w, normPart, (const Scalars *)sc);
         }
-        hipLaunchKernelGGL(kGmGivens, dim3(1), dim3(kFinBlock), 0, st, j, ld, (const double *)normPart, G, H, cs,
+        hipLaunchKernelGGL(kGmGivens, dim3(1), dim3(kFinBlock), 0, st, j, ld, (const double *)normPart, Ga, H, cs,
                            sn, g, vscale, sc);
         hipLaunchKernelGGL((kGmScale<T>), dim3(ge), dim3(256), 0, st, n, w, (const double *)vscale,
                            (const Scalars *)sc);
