@@ -15,6 +15,8 @@ struct phase_hip_equation {
   phase::DBuf<int> cols, cnt;
   phase::DBuf<double> vals, rhs;
   phase::DBuf<int> dErr;
+  int *hErr = nullptr;   // a pinned slot: where dErr is read to
   bool compact = false;  // rows rebuilt by += / -= (no empty slots)
   std::string err;
+  ~phase_hip_equation();
 };

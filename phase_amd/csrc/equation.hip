@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -1145,11 +1146,48 @@ int guardedM(phase_hip_mesh *m, F &&f) {
   }
 }
 
+// Pinned ints for the equations' error bits, one block of 1024 for the process
+// (a pinned allocation per equation took longer than the rest of its creation);
+// past those, an allocation of its own.
+class PinnedSlots {
+ public:
+  int *take() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (!block_) {
+      PH_CHECK(hipHostMalloc((void **)&block_, kSlots * sizeof(int), hipHostMallocPortable));
+      for (int i = 0; i < kSlots; ++i) free_.push_back(block_ + i);
+    }
+    int *p = nullptr;
+    if (free_.empty()) {
+      PH_CHECK(hipHostMalloc((void **)&p, sizeof(int), hipHostMallocPortable));
+    } else {
+      p = free_.back();
+      free_.pop_back();
+    }
+    return p;
+  }
+  void give(int *p) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (p >= block_ && p < block_ + kSlots) free_.push_back(p);
+    else (void)hipHostFree(p);
+  }
+
+ private:
+  static constexpr int kSlots = 1024;
+  std::mutex mutex_;
+  int *block_ = nullptr;
+  std::vector<int *> free_;
+};
+PinnedSlots &pinnedSlots() {
+  static PinnedSlots *s = new PinnedSlots();  // never destroyed: equations may outlive static objects
+  return *s;
+}
+
 // Device error bits of the last operator: raised as the reference's exceptions.
 void checkEq(phase_hip_equation *e, const char *op) {
-  int v = 0;
-  PH_CHECK(hipMemcpyAsync(&v, e->dErr.p, sizeof(int), hipMemcpyDeviceToHost, e->mesh->stream));
+  PH_CHECK(hipMemcpyAsync(e->hErr, e->dErr.p, sizeof(int), hipMemcpyDeviceToHost, e->mesh->stream));
   PH_CHECK(hipStreamSynchronize(e->mesh->stream));
+  const int v = *e->hErr;
   if (!v) return;
   PH_CHECK(hipMemsetAsync(e->dErr.p, 0, sizeof(int), e->mesh->stream));
   if (v & 1) fail(PHASE_HIP_EBOUNDARY, std::string(op) + ": unrecognized or unspecified boundary type.");
@@ -1160,6 +1198,10 @@ void checkEq(phase_hip_equation *e, const char *op) {
 void fresh(phase_hip_equation *e) { e->compact = false; }
 
 }  // namespace
+
+phase_hip_equation::~phase_hip_equation() {
+  if (hErr) pinnedSlots().give(hErr);
+}
 
 namespace phase {
 
@@ -1196,6 +1238,7 @@ int phase_hip_equation_create(phase_hip_equation **out, phase_hip_mesh *m, int n
     e->rhs.alloc(e->rank);
     e->dErr.alloc(1);
     e->dErr.zero(m->stream);
+    e->hErr = pinnedSlots().take();
     // CrsEquation(N, 5): every slot empty
     PH_CHECK(hipMemsetAsync(e->cols.p, 0xff, slots * sizeof(int), m->stream));
     e->vals.zero(m->stream);

@@ -25,6 +25,7 @@
 #include "mesh.h"
 #include "solver.h"
 #include "solver_kernels.h"
+#include "solver_launch.h"
 
 using namespace phase;
 
@@ -611,9 +612,7 @@ namespace phase {
 void checkAssembly(phase_hip_solver *s) {
   if (!s->binding) return;
   MeshBinding &b = *s->binding;
-  int e = 0;
-  PH_CHECK(hipMemcpyAsync(&e, b.dErr.p, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-  PH_CHECK(hipStreamSynchronize(s->stream));
+  const int e = pullValue(s, b.dErr.p);
   if (e) {
     b.dErr.zero(s->stream);
     fail(PHASE_HIP_EBOUNDARY, "fv::laplacian: unrecognized or unspecified boundary type.");

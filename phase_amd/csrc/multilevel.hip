@@ -455,33 +455,31 @@ __global__ __launch_bounds__(kGjBlock) void kDenseInverseDiag(int n, const doubl
 // Largest n the register Gauss-Jordan kernels take (RB = 6: 36 entries per thread).
 constexpr int kDenseRegMax = 192;
 
-// inv = dense^-1 into `inv`; err bit 4 on a singular matrix.  Up to
+// inv = dense^-1 into `inv`; returns the error bits (4: singular matrix).  Up to
 // kDenseRegMax rows, without pivoting first unless `pivot`, and with pivoting
 // when that flags a small pivot (one host synchronisation each).
-void denseInverse(hipStream_t st, int n, double *dense, double *inv, int *err, bool pivot) {
-  auto readErr = [&] {
-    int e = 0;
-    PH_CHECK(hipMemcpyAsync(&e, err, sizeof(int), hipMemcpyDeviceToHost, st));
-    PH_CHECK(hipStreamSynchronize(st));
-    return e;
-  };
+int denseInverse(phase_hip_solver *s, int n, double *dense, double *inv, bool pivot) {
+  hipStream_t st = s->stream;
+  int *err = s->dErr.p;
   if (n > kDenseRegMax) {
     hipLaunchKernelGGL(kDenseInverse, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
     PH_CHECK(hipGetLastError());
-    return;
+    return pullValue(s, err);
   }
   if (!pivot) {
     if (n <= 64) hipLaunchKernelGGL(kDenseInverseDiag<2>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
     else if (n <= 128) hipLaunchKernelGGL(kDenseInverseDiag<4>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
     else hipLaunchKernelGGL(kDenseInverseDiag<6>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
     PH_CHECK(hipGetLastError());
-    if (!(readErr() & 8)) return;
+    const int e = pullValue(s, err);
+    if (!(e & 8)) return e;
     PH_CHECK(hipMemsetAsync(err, 0, sizeof(int), st));
   }
   if (n <= 64) hipLaunchKernelGGL(kDenseInverseReg<2>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
   else if (n <= 128) hipLaunchKernelGGL(kDenseInverseReg<4>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
   else hipLaunchKernelGGL(kDenseInverseReg<6>, dim3(1), dim3(kGjBlock), 0, st, n, dense, inv, err);
   PH_CHECK(hipGetLastError());
+  return pullValue(s, err);
 }
 
 // e = inv r (one wavefront per row, FP64 products)
@@ -1556,11 +1554,8 @@ void mlEnsureValues(phase_hip_solver *s, bool single) {
                            finer, L.cVals.p);
         hipLaunchKernelGGL(kDenseFill, dim3(elemGrid(L.n)), dim3(256), 0, st, L.n, L.cRowPtr.p, L.cColInd.p,
                            L.cVals.p, L.dense.p);
-        denseInverse(st, L.n, L.dense.p, L.inv.p, s->dErr.p, s->mlDensePivot != 0);
+        const int e = denseInverse(s, L.n, L.dense.p, L.inv.p, s->mlDensePivot != 0);
         hipLaunchKernelGGL(kTransposeDense, dim3(elemGrid((long)L.n * L.n)), dim3(256), 0, st, L.n, L.inv.p, L.invT.p);
-        int e = 0;
-        PH_CHECK(hipMemcpyAsync(&e, s->dErr.p, sizeof(int), hipMemcpyDeviceToHost, st));
-        PH_CHECK(hipStreamSynchronize(st));
         if (e & 4) {
           PH_CHECK(hipMemsetAsync(s->dErr.p, 0, sizeof(int), st));
           fail(PHASE_HIP_EBREAKDOWN, "multigrid: singular coarsest matrix");

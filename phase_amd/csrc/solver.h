@@ -95,7 +95,7 @@ struct phase_hip_solver {
   phase::DBuf<double> dPartials;
   phase::DBuf<unsigned> dCounter;
   phase::DBuf<phase::Scalars> dSc;  // [0] inner run, [1] outer residual, [2] misc
-  phase::Scalars *hSc = nullptr;    // pinned mirror of dSc
+  phase::Scalars *hSc = nullptr;    // pinned mirror of dSc's first three, and a slot for single values
   phase::DBuf<double> dMisc;        // [0] ||b||^2
 
   // results of the last solve

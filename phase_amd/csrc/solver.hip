@@ -164,11 +164,10 @@ double normB2(phase_hip_solver *s) {
   const int g = gridFor(n, kRedBlock, kRedCap);
   hipLaunchKernelGGL((kNorm2<double>), dim3(g), dim3(kRedBlock), 0, s->stream, n, s->dB.p, s->dPartials.p);
   hipLaunchKernelGGL(kFinishNorm2, dim3(1), dim3(kFinBlock), 0, s->stream, s->dPartials.p, g, s->dMisc.p);
-  double b2 = 0.;
-  PH_CHECK(hipMemcpyAsync(&b2, s->dMisc.p, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-  PH_CHECK(hipStreamSynchronize(s->stream));
-  return b2;
+  return pullValue(s, s->dMisc.p);
 }
+
+bool capturing(phase_hip_solver *s) { return s->gnn && s->gnn->captureEvery > 0; }
 
 // Run Krylov chunks until the device says done; returns iterations taken.
 // onChunk(iterationsSoFar) runs on the host after every chunk and returns
@@ -176,13 +175,19 @@ double normB2(phase_hip_solver *s) {
 // the threshold still launch (each returns at once), so once a rate is known
 // the next chunk is the number of iterations the last chunk's rate of
 // decrease needs to reach the threshold (at most `chunk`): a guess one short
-// costs a host round trip, one long an iteration of empty launches.
+// costs a host round trip, one long an iteration of empty launches.  The first
+// chunk is two iterations, whose rate from the starting residual (the caller has
+// pulled it into hSc[0]) serves the same: equations dominated by their diagonal
+// (momentum, volume fraction) converge in three or four, and four or five more
+// queued cost 16 launches of 2 to 3 us each.  While pairs are captured, whose
+// snapshots fall on chunk ends, it is `chunk`.
+constexpr int kFirstChunk = 2;
 template <class T, class TX, class TV, class OnChunk>
 int runKrylov(phase_hip_solver *s, KrylovVecs<T> &K, DBuf<T> &fac, const TV *sell, TX *x, int budget,
               OnChunk &&onChunk) {
   Scalars *sc = s->dSc.p;  // slot 0
-  int it = 0, chunk = s->chunk, itLast = 0;
-  double rrLast = -1.;
+  int it = 0, chunk = capturing(s) ? s->chunk : std::min(s->chunk, kFirstChunk), itLast = 0;
+  double rrLast = s->hSc[0].rr;
   while (true) {
     for (int c = 0; c < chunk; ++c) {
       if (s->cg) iterateCg<T, TX, TV>(s, K, fac, sell, x, sc);
@@ -202,11 +207,8 @@ int runKrylov(phase_hip_solver *s, KrylovVecs<T> &K, DBuf<T> &fac, const TV *sel
     rrLast = h.rr;
     itLast = it;
   }
-  checkDeviceErr(s);
   return it;
 }
-
-bool capturing(phase_hip_solver *s) { return s->gnn && s->gnn->captureEvery > 0; }
 
 // FP64 BiCGStab + ILU(0) from the current x.  `total` iterations were already
 // spent by the caller (a mixed solve falling back); the loop restarts the
@@ -437,7 +439,7 @@ void allocCommon(phase_hip_solver *s) {
   s->dSc.alloc(4);  // [3]: idle slot, done == 0, for sweeps outside a Krylov run
   s->dSc.zero(s->stream);
   s->dMisc.alloc(4);
-  if (!s->hSc) PH_CHECK(hipHostMalloc((void **)&s->hSc, 3 * sizeof(Scalars), hipHostMallocDefault));
+  if (!s->hSc) PH_CHECK(hipHostMalloc((void **)&s->hSc, 4 * sizeof(Scalars), hipHostMallocDefault));
 }
 
 }  // namespace
@@ -551,10 +553,7 @@ void solverSetFromRows(phase_hip_solver *s, int rank, int stride, const int *dCo
     s->dEqFlag.zero(s->stream);
     hipLaunchKernelGGL(kCmpInt, dim3(gridFor((long)slots, 256, kElemCap)), dim3(256), 0, s->stream, slots, dCols,
                        s->dEqCols.p, s->dEqFlag.p);
-    int flag = 0;
-    PH_CHECK(hipMemcpyAsync(&flag, s->dEqFlag.p, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    PH_CHECK(hipStreamSynchronize(s->stream));
-    same = flag == 0;
+    same = pullValue(s, s->dEqFlag.p) == 0;
   }
   // union patterns: a pattern inside the stored one keeps the ordering and
   // factor structure, with explicit zeros for the entries it lacks
@@ -565,10 +564,7 @@ void solverSetFromRows(phase_hip_solver *s, int rank, int stride, const int *dCo
     s->dEqFlag.zero(s->stream);
     hipLaunchKernelGGL(kSubsetCols, dim3(gridFor(rank, 256, kElemCap)), dim3(256), 0, s->stream, rank, stride, dCols,
                        s->eqStride, s->dEqCols.p, s->dEqFlag.p);
-    int flag = 0;
-    PH_CHECK(hipMemcpyAsync(&flag, s->dEqFlag.p, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    PH_CHECK(hipStreamSynchronize(s->stream));
-    remap = flag == 0;
+    remap = pullValue(s, s->dEqFlag.p) == 0;
   }
   if (!same && !remap) {
     std::vector<int> cols(slots), rowPtr(rank + 1);

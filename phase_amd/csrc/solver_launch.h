@@ -1,5 +1,5 @@
-// Launchers shared by the solver and the multigrid hierarchy (included by
-// solver.hip and multilevel.hip only): grid sizes, the ILU(0) sweeps and
+// Launchers shared by the solver and the multigrid hierarchy (included by the
+// files that run solver kernels): grid sizes, the ILU(0) sweeps and
 // factorisation of one ordering, and the lazily built FP64 / FP32 factors.
 #pragma once
 
@@ -122,10 +122,19 @@ inline void pullScalars(phase_hip_solver *s) {
   PH_CHECK(hipStreamSynchronize(s->stream));
 }
 
-inline void checkDeviceErr(phase_hip_solver *s) {
-  int e = 0;
-  PH_CHECK(hipMemcpyAsync(&e, s->dErr.p, sizeof(int), hipMemcpyDeviceToHost, s->stream));
+// One value of the device to the host.  By way of the handle's pinned memory: a
+// copy to a variable on the stack is staged by the runtime and takes the host
+// about twice as long.
+template <class T>
+T pullValue(phase_hip_solver *s, const T *d) {
+  static_assert(sizeof(T) <= sizeof(Scalars), "the slot behind the three records");
+  PH_CHECK(hipMemcpyAsync(s->hSc + 3, d, sizeof(T), hipMemcpyDeviceToHost, s->stream));
   PH_CHECK(hipStreamSynchronize(s->stream));
+  return *reinterpret_cast<const T *>(s->hSc + 3);
+}
+
+inline void checkDeviceErr(phase_hip_solver *s) {
+  const int e = pullValue(s, s->dErr.p);
   if (e & 2) {
     PH_CHECK(hipMemsetAsync(s->dErr.p, 0, sizeof(int), s->stream));
     fail(PHASE_HIP_EBREAKDOWN, "zero pivot in ILU(0) factorisation");
