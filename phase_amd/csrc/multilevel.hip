@@ -31,7 +31,7 @@ struct MlVecs {
   }
   // the finest level uses the cycle work vectors only
   void allocCycle(int n) {
-    for (DBuf<T> *b : {&t, &w, &y}) b->alloc(n);
+    for (DBuf<T> *b : {&t, &w, &y, &u}) b->alloc(n);
   }
 };
 
@@ -51,6 +51,8 @@ struct MlLevel {
   DBuf<int> restRow;                // this level's solver row -> aggregate of the finer level (dense: identity)
   DBuf<int> finerAggPtr;            // finer solver rows of each aggregate
   DBuf<int> pIdx;                   // finer solver row -> this level's solver row
+  DBuf<int> groupAgg;               // first coarse level: runs of aggregates of at most kRunRows rows
+  int nGroups = 0;
   int nFiner = 0, nSlots = 0;
   // dense last level
   DBuf<int> cRowPtr, cColInd;
@@ -510,28 +512,6 @@ __global__ __launch_bounds__(kRedBlock) void kMlResid(int n, int nSlices, const 
   t[row] = b[row] - sellRow<T, TV>(slice, lane, sliceOff, col, val, x);
 }
 
-// rc[k] = sum of t over the finer rows of aggregate restRow[k] (identity when
-// null; an aggregate's rows are consecutive in the finer solver order), in
-// FP64: 16 lanes per coarse row, lane l summing rows l, l + 16, ... in order,
-// then a fixed xor tree over the 16 lanes (one or two load rounds for an
-// aggregate of about 32 rows, where a thread per aggregate took seven).
-template <class T>
-__global__ __launch_bounds__(256) void kMlRestrictRows(int nc, const int *__restrict__ restRow,
-                                                       const int *__restrict__ aggPtr, const T *__restrict__ t,
-                                                       T *__restrict__ rc, const Scalars *sc) {
-  if (sc->done) return;
-  const int k = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;
-  double d = 0.;
-  if (k < nc) {
-    const int a = restRow ? restRow[k] : k;
-    const int r1 = aggPtr[a + 1];
-    for (int i = aggPtr[a] + l; i < r1; i += 16) d += (double)t[i];
-  }
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) d += __shfl_xor(d, o, 16);
-  if (k < nc && l == 0) rc[k] = (T)d;
-}
-
 // e[i] += ec[pIdx[i]]
 template <class T>
 __global__ void kMlProlongAdd(int n, const int *__restrict__ pIdx, const T *__restrict__ ec, T *__restrict__ e,
@@ -542,8 +522,10 @@ __global__ void kMlProlongAdd(int n, const int *__restrict__ pIdx, const T *__re
 
 // Row `row` of A x in SELL-64 for a lane whose slice need not be the rest of
 // the wavefront's: the products and their order are sellRow's (x[c] comes
-// from gx(c)), so the result is bit-identical to it.
-template <class T, class TV, class GX>
+// from gx(c)), so the result is bit-identical to it.  STREAM: the finest level,
+// whose matrix does not stay in L2 (non-temporal loads, as sellRow's), with
+// eight entries' loads in flight.
+template <class T, class TV, bool STREAM = false, class GX>
 __device__ __forceinline__ T sellRowAt(int row, const int *__restrict__ sliceOff, const int *__restrict__ col,
                                        const TV *__restrict__ val, GX &&gx) {
   using A = typename std::conditional<(sizeof(TV) > sizeof(T)), TV, T>::type;
@@ -551,22 +533,23 @@ __device__ __forceinline__ T sellRowAt(int row, const int *__restrict__ sliceOff
   const int o = sliceOff[slice];
   const int K = (sliceOff[slice + 1] - o) >> 6;
   A acc = 0;
-  for (int e0 = 0; e0 < K; e0 += 4) {
-    int c[4];
-    TV a[4];
+  constexpr int N = STREAM ? kSellBatch : 4;
+  for (int e0 = 0; e0 < K; e0 += N) {
+    int c[N];
+    TV a[N];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < N; ++q)
       if (e0 + q < K) {
         const int idx = o + ((e0 + q) << 6) + lane;
-        c[q] = col[idx];
-        a[q] = val[idx];
+        c[q] = STREAM ? __builtin_nontemporal_load(col + idx) : col[idx];
+        a[q] = STREAM ? __builtin_nontemporal_load(val + idx) : val[idx];
       }
-    T xv[4];
+    T xv[N];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < N; ++q)
       if (e0 + q < K) xv[q] = gx(c[q] >= 0 ? c[q] : 0);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < N; ++q)
       if (e0 + q < K && c[q] >= 0) acc = fma((A)a[q], (A)xv[q], acc);
   }
   return (T)acc;
@@ -597,10 +580,47 @@ __global__ __launch_bounds__(256) void kMlResidRestrict(int nc, const int *__res
   if (lane == 0) rc[k] = (T)d;
 }
 
-// Coarse levels, kMlProlongAdd and kMlResid in one launch:
+// The finest level's residual and restriction in one launch: a workgroup takes
+// a run of whole aggregates of at most 256 rows (groupAgg, built with the
+// hierarchy), one row per thread, leaves the residuals in LDS and sums them there.  Bound by HBM as kMlResid is; the residual vector is
+// neither written nor read.  A row's residual is rounded to T before the FP64
+// sum; 16 lanes per aggregate, lane l summing rows l, l + 16, ... in order, then a
+// fixed xor tree over the 16 lanes.  One million triangles, FP32 vectors: 15.6 us
+// (as two launches 13.5 + 5.0); two million quads, FP64: 32.8 us (28.4 + 7.7).
+constexpr int kRunRows = 256;
+template <class T, class TV>
+__global__ __launch_bounds__(kRunRows) void kMlResidRestrictRuns(const int *__restrict__ groupAgg,
+                                                                 const int *__restrict__ aggPtr,
+                                                                 const int *__restrict__ pIdx,
+                                                                 const int *__restrict__ sliceOff,
+                                                                 const int *__restrict__ col,
+                                                                 const TV *__restrict__ val,
+                                                                 const T *__restrict__ x, const T *__restrict__ b,
+                                                                 T *__restrict__ rc, const Scalars *sc) {
+  if (sc->done) return;
+  __shared__ T ts[kRunRows];
+  const int g = xcdTile(blockIdx.x, gridDim.x);
+  const int a0 = groupAgg[g], a1 = groupAgg[g + 1];
+  const int r0 = aggPtr[a0], row = r0 + threadIdx.x;
+  if (row < aggPtr[a1])
+    ts[threadIdx.x] = b[row] - sellRowAt<T, TV, true>(row, sliceOff, col, val, [&](int c) { return x[c]; });
+  __syncthreads();
+  const int l = threadIdx.x & 15;
+  for (int a = a0 + (threadIdx.x >> 4); a < a1; a += kRunRows / 16) {
+    const int i0 = aggPtr[a], i1 = aggPtr[a + 1];
+    double d = 0.;
+    for (int i = i0 + l; i < i1; i += 16) d += (double)ts[i - r0];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) d += __shfl_xor(d, o, 16);
+    if (l == 0) rc[pIdx[i0]] = (T)d;
+  }
+}
+
+// kMlProlongAdd and kMlResid in one launch:
 // u = z + P ec and t = b - A u, where A's products read z + P ec at the
 // gathered columns (the sums kMlProlongAdd would store) and z stays as it is.
-template <class T, class TV>
+// FINE: the finest level.
+template <class T, class TV, bool FINE = false>
 __global__ __launch_bounds__(kRedBlock) void kMlResidProlong(int n, int nSlices, const int *__restrict__ sliceOff,
                                                              const int *__restrict__ col, const TV *__restrict__ val,
                                                              const int *__restrict__ pIdx,
@@ -608,10 +628,11 @@ __global__ __launch_bounds__(kRedBlock) void kMlResidProlong(int n, int nSlices,
                                                              const T *__restrict__ b, T *__restrict__ t,
                                                              T *__restrict__ u, const Scalars *sc) {
   if (sc->done) return;
-  const int slice = blockIdx.x * (kRedBlock / 64) + (threadIdx.x >> 6);
+  const int tile = FINE ? xcdTile(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int slice = tile * (kRedBlock / 64) + (threadIdx.x >> 6);
   const int row = slice * 64 + (threadIdx.x & 63);
   if (slice >= nSlices || row >= n) return;
-  const T y = sellRowAt<T, TV>(row, sliceOff, col, val, [&](int c) { return (T)(z[c] + ec[pIdx[c]]); });
+  const T y = sellRowAt<T, TV, FINE>(row, sliceOff, col, val, [&](int c) { return (T)(z[c] + ec[pIdx[c]]); });
   t[row] = b[row] - y;
   u[row] = z[row] + ec[pIdx[row]];
 }
@@ -1294,29 +1315,20 @@ void coarseSolve(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, c
   hipLaunchKernelGGL((kMlSecond<T>), dim3(gd), dim3(kRedBlock), 0, st, n, sc, L.partials.p, gs, V.z2.p, e);
 }
 
-// Restriction of the residual t (finer solver order) into level l's
-// right-hand side, the coarse solve, and the prolongation added to z.
-template <class T>
-void coarseCorrection(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *t, T *z) {
-  MlLevel &L = M.lv[l];
-  MlVecs<T> &V = vecs<T>(L);
-  hipStream_t st = s->stream;
-  hipLaunchKernelGGL((kMlRestrictRows<T>), dim3((L.n + 15) / 16), dim3(256), 0, st, L.n,
-                     L.sol ? L.restRow.p : nullptr, L.finerAggPtr.p, t, V.r.p, sc);
-  coarseSolve<T>(s, M, l, sc, V.r.p, V.e.p);
-  hipLaunchKernelGGL((kMlProlongAdd<T>), dim3(elemGrid(L.nFiner)), dim3(256), 0, st, L.nFiner, L.pIdx.p,
-                     (const T *)V.e.p, z, sc);
-}
-
 // Smoothing, coarse correction and smoothing at level `lvl` (nested solver c,
 // its work vectors V): z = B r.  When `pre` is false the pre-smoothing has
 // already put M^-1 r into z.
 //
-// On the coarse levels (c nested), where every launch costs more than its
-// arithmetic, the residual and its restriction run as one launch, and so do
-// the prolongation and the post-smoothing residual (into the work vector u);
-// at every level the post-smoothing sweep adds its result into z as it
-// finishes each row.  The arithmetic is that of the separate kernels.
+// The residual and its restriction run as one launch, and so do the
+// prolongation and the post-smoothing residual (into the work vector u): on the
+// coarse levels (c nested) every launch costs more than its arithmetic, on the
+// finest the first saves a pass over the residual.  The second gathers the coarse
+// row and its correction with every entry, which on a large finest level takes
+// longer than the pass and the launch it saves (FP32 vectors: 4.9 us against 7.0
+// at 16,384 rows, 7.6 against 8.7 at 200,000, 20.5 against 18.1 at one million): the line
+// is drawn at kFusedProlongRows.  The post-smoothing sweep adds its result into z
+// as it finishes each row.  The arithmetic is that of the separate kernels.
+constexpr int kFusedProlongRows = 1 << 18;
 template <class T>
 void smoothCorrectSmooth(phase_hip_solver *s, Multilevel &M, phase_hip_solver *c, MlVecs<T> &V, int next,
                          const Scalars *sc, const T *r, T *z, bool pre, bool post = true) {
@@ -1339,14 +1351,27 @@ void smoothCorrectSmooth(phase_hip_solver *s, Multilevel &M, phase_hip_solver *c
                           nullptr, (const T *)V.u.p, z);
     return;
   }
-  hipLaunchKernelGGL((kMlResid<T, double>), dim3(gs), dim3(kRedBlock), 0, st, n, c->ord.nSlices, c->dSliceOff.p,
-                     c->dSellCol.p, c->dSell64.p, (const T *)z, r, V.t.p, sc);
-  coarseCorrection<T>(s, M, next, sc, V.t.p, z);
-  if (!post) return;
-  hipLaunchKernelGGL((kMlResid<T, double>), dim3(gs), dim3(kRedBlock), 0, st, n, c->ord.nSlices, c->dSliceOff.p,
-                     c->dSellCol.p, c->dSell64.p, (const T *)z, r, V.t.p, sc);
+  MlLevel &N = M.lv[next];
+  MlVecs<T> &NV = vecs<T>(N);
+  hipLaunchKernelGGL((kMlResidRestrictRuns<T, double>), dim3(N.nGroups), dim3(kRunRows), 0, st, N.groupAgg.p,
+                     N.finerAggPtr.p, N.pIdx.p, c->dSliceOff.p, c->dSellCol.p, c->dSell64.p, (const T *)z, r, NV.r.p,
+                     sc);
+  coarseSolve<T>(s, M, next, sc, NV.r.p, NV.e.p);
+  if (!post || n > kFusedProlongRows) {
+    hipLaunchKernelGGL((kMlProlongAdd<T>), dim3(elemGrid(n)), dim3(256), 0, st, n, N.pIdx.p, (const T *)NV.e.p, z,
+                       sc);
+    if (!post) return;
+    hipLaunchKernelGGL((kMlResid<T, double>), dim3(gs), dim3(kRedBlock), 0, st, n, c->ord.nSlices, c->dSliceOff.p,
+                       c->dSellCol.p, c->dSell64.p, (const T *)z, r, V.t.p, sc);
+    launchLU<T, kProNone>(c, L, sc, V.t.p, V.y.p, (T *)nullptr, (const T *)nullptr, (const T *)nullptr, V.w.p,
+                          nullptr, (const T *)z, z);
+    return;
+  }
+  hipLaunchKernelGGL((kMlResidProlong<T, double, true>), dim3(gs), dim3(kRedBlock), 0, st, n, c->ord.nSlices,
+                     c->dSliceOff.p, c->dSellCol.p, c->dSell64.p, N.pIdx.p, (const T *)NV.e.p, (const T *)z, r, V.t.p,
+                     V.u.p, sc);
   launchLU<T, kProNone>(c, L, sc, V.t.p, V.y.p, (T *)nullptr, (const T *)nullptr, (const T *)nullptr, V.w.p,
-                        nullptr, (const T *)z, z);
+                        nullptr, (const T *)V.u.p, z);
 }
 
 template <class T>
@@ -1452,6 +1477,15 @@ void mlEnsureHierarchy(phase_hip_solver *s) {
       L.galPtr.upload(c.galPtr, st);
       L.galSrc.upload(c.galSrc.empty() ? std::vector<int>{0} : c.galSrc, st);
       L.finerAggPtr.upload(fine->aggPtr, st);
+      if (level == 0) {
+        std::vector<int> runs(1, 0);
+        for (int a = 0; a < c.n; ++a)
+          if (fine->aggPtr[a + 1] - fine->aggPtr[runs.back()] > kRunRows) runs.push_back(a);
+        L.nGroups = (int)runs.size();
+        runs.push_back(c.n);
+        L.groupAgg.upload(runs, st);
+        PH_CHECK(hipStreamSynchronize(st));  // before `runs` goes
+      }
       std::vector<int> pIdx(nFiner);
       bool dense = c.n <= s->mlDenseRows;
       if (!dense) {
