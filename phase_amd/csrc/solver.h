@@ -70,6 +70,7 @@ struct phase_hip_solver {
   std::vector<double> cellXY;  // row centroids of the pattern (brick aggregates), empty when unknown
   std::vector<int> patRowPtr, patColInd;
   phase::Ordering ord;
+  int facSlots = 1;  // entries per row the factorisation holds in LDS (the widest block's)
 
   phase::DBuf<phase::BlockInfo> dBlocks;
   phase::DBuf<phase::RowInfo> dRows;

@@ -173,15 +173,6 @@ __device__ void finishPartials(const double *partials, int nb, double (&v)[NV]) 
 }
 
 // ---------------------------------------------------------------- data movement
-template <class T>
-__global__ void kGather(int m, const int *__restrict__ map, const double *__restrict__ src,
-                        T *__restrict__ dst) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) {
-    const int s = map[i];
-    dst[i] = s >= 0 ? (T)src[s] : (T)0;
-  }
-}
-
 // out[k] = in[perm[k]] (original -> solver order)
 template <class TI, class TO>
 __global__ void kPermuteIn(int n, const int *__restrict__ perm, const TI *__restrict__ in,
@@ -644,34 +635,138 @@ __device__ __forceinline__ int colourBlock(int blockBase) { return blockBase + x
 // (i,k) in ascending k: l = a_ik / u_kk, then a_ij -= l * u_kj over U(k) in
 // ascending j.  Rows of earlier blocks are final (earlier colour launch); rows
 // of the same block are final after their level.  A zero pivot sets bit 2 of
-// *err.
+// *err.  A block takes its entries straight from the matrix values (facSrc; -1:
+// zero) and writes its slots, pads as zeros, and the inverse diagonal.
+// Bound by the chain of levels.  The block's entries are held in LDS
+// (L slots | U slots | diagonal), and before the levels a row loads what it
+// needs of earlier blocks, final by then: the pivots of its first kFacW
+// entries and the sources of their first two updates each.  A level then costs
+// divisions and LDS trips, where in global memory each entry was a chain of
+// round trips.  One million quads (FP64, 4 colours, 32,849 blocks): 199 us for
+// the factorisation, 427 with the entries gathered by a launch of its own, the
+// updates in global memory and the inverse diagonal in a third launch (97 + 330
+// + 7); 500,000 quads (3 colours) 62 against 153; 16,384 quads 11.8 us a colour, 19.7.
+constexpr int kFacW = 4;
+extern __shared__ __align__(16) char facStage[];
 template <class T>
-__global__ __launch_bounds__(64) void kIluFactor(IluDev<T> L, const int *__restrict__ updPtr,
+__global__ __launch_bounds__(64) void kIluFactor(IluDev<T> L, int n, const double *__restrict__ vals,
+                                                 const int *__restrict__ facSrc, const int *__restrict__ updPtr,
                                                  const int *__restrict__ updSrc,
                                                  const int *__restrict__ updDst, int *err, int blockBase) {
+  T *f = (T *)facStage;
   const int b = colourBlock(blockBase);
   const BlockInfo B = L.blocks[b];
   const int lane = threadIdx.x;
   const bool act = lane < B.nRows;
   const int row = B.rowStart + lane;
   const RowInfo ri = act ? L.rows[row] : RowInfo{};
+  const int nL = act ? ri.nL : 0;
+  const int dbase = L.nLSlots + L.nUSlots, uFirst = L.nLSlots + B.uOff;
   T *fac = L.fac;
-  const int dbase = L.nLSlots + L.nUSlots;
+  // place of an entry of this block in LDS; -1: an earlier block's
+  auto place = [&](int s) {
+    if (s < L.nLSlots) return s - B.lOff;  // L entries are only read and written by their own row
+    if (s < dbase) return s >= uFirst && s < uFirst + (B.kU << 6) ? (B.kL << 6) + s - uFirst : -1;
+    return s - dbase >= B.rowStart && s - dbase < B.rowStart + B.nRows ? ((B.kL + B.kU) << 6) + s - dbase - B.rowStart
+                                                                      : -1;
+  };
+  const int nSlot = B.kL + B.kU, dAt = (nSlot << 6) + lane;
+  const int *lSrc = facSrc + B.lOff + lane, *uSrc = facSrc + uFirst + lane - (B.kL << 6);
+  for (int e0 = 0; e0 <= nSlot; e0 += 4) {  // four entries at a time, the diagonal as the last
+    int at[4];
+    double x[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int e = e0 + c;
+      at[c] = -1;
+      if (e < nSlot) at[c] = (e < B.kL ? lSrc : uSrc)[e << 6];
+      else if (e == nSlot && act) at[c] = facSrc[dbase + row];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) x[c] = at[c] >= 0 ? vals[at[c]] : 0.0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (e0 + c <= nSlot) f[((e0 + c) << 6) + lane] = (T)x[c];
+  }
+  // the first entries' pivots and updates
+  int pAt[kFacW], p0[kFacW], p1[kFacW], sAt[kFacW][2], tAt[kFacW][2];
+  T pv[kFacW], sv[kFacW][2];
+#pragma unroll
+  for (int e = 0; e < kFacW; ++e) {
+    pAt[e] = p0[e] = p1[e] = 0;
+    if (e < nL) {
+      const int s = B.lOff + (e << 6) + lane;
+      pAt[e] = dbase + L.lCol[s];
+      p0[e] = updPtr[s];
+      p1[e] = updPtr[s + 1];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < kFacW; ++e)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      sAt[e][u] = tAt[e][u] = 0;
+      if (p0[e] + u < p1[e]) {
+        sAt[e][u] = updSrc[p0[e] + u];
+        tAt[e][u] = updDst[p0[e] + u];
+      }
+    }
+#pragma unroll
+  for (int e = 0; e < kFacW; ++e) {
+    pv[e] = 1;
+    if (e < nL) {
+      const int at = place(pAt[e]);
+      if (at < 0) pv[e] = fac[pAt[e]];
+      pAt[e] = at;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      sv[e][u] = 0;
+      if (p0[e] + u < p1[e]) {
+        const int at = place(sAt[e][u]);
+        if (at < 0) sv[e][u] = fac[sAt[e][u]];
+        sAt[e][u] = at;
+        tAt[e][u] = place(tAt[e][u]);
+      }
+    }
+  }
+  __syncthreads();
   for (int lev = 0; lev < B.nLev; ++lev) {
     if (act && ri.lev == lev) {
-      for (int e = 0; e < ri.nL; ++e) {
-        const int s = B.lOff + (e << 6) + lane;
-        const int k = L.lCol[s];
-        const T lik = fac[s] / fac[dbase + k];
-        fac[s] = lik;
+#pragma unroll
+      for (int e = 0; e < kFacW; ++e)
+        if (e < nL) {
+          const T lik = f[(e << 6) + lane] / (pAt[e] >= 0 ? f[pAt[e]] : pv[e]);
+          f[(e << 6) + lane] = lik;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            if (p0[e] + u < p1[e]) {
+              const T src = sAt[e][u] >= 0 ? f[sAt[e][u]] : sv[e][u];
+              f[tAt[e][u]] = fma(-lik, src, f[tAt[e][u]]);
+            }
+          for (int u = p0[e] + 2; u < p1[e]; ++u) {
+            const int at = place(updSrc[u]), to = place(updDst[u]);
+            f[to] = fma(-lik, at >= 0 ? f[at] : fac[updSrc[u]], f[to]);
+          }
+        }
+      for (int e = kFacW; e < nL; ++e) {
+        const int s = B.lOff + (e << 6) + lane, k = dbase + L.lCol[s], at = place(k);
+        const T lik = f[(e << 6) + lane] / (at >= 0 ? f[at] : fac[k]);
+        f[(e << 6) + lane] = lik;
         for (int u = updPtr[s]; u < updPtr[s + 1]; ++u) {
-          const int dst = updDst[u];
-          fac[dst] = fma(-lik, fac[updSrc[u]], fac[dst]);
+          const int from = place(updSrc[u]), to = place(updDst[u]);
+          f[to] = fma(-lik, from >= 0 ? f[from] : fac[updSrc[u]], f[to]);
         }
       }
-      if (fac[dbase + row] == (T)0) atomicOr(err, 2);
+      if (f[dAt] == (T)0) atomicOr(err, 2);
     }
     __syncthreads();
+  }
+  for (int e = 0; e < B.kL; ++e) fac[B.lOff + (e << 6) + lane] = f[(e << 6) + lane];
+  for (int e = 0; e < B.kU; ++e) fac[uFirst + (e << 6) + lane] = f[((B.kL + e) << 6) + lane];
+  if (act) {
+    fac[dbase + row] = f[dAt];
+    fac[dbase + n + row] = (T)1 / f[dAt];  // read by the backward sweep
   }
 }
 
@@ -689,13 +784,6 @@ __global__ __launch_bounds__(64) void kIluFactor(IluDev<T> L, const int *__restr
 // the registers (coarse multigrid levels) keep the array.  The fused launch over
 // 7,168 rows takes 4.5 us in FP32 (6.4 us with the array), 27,264 rows in FP64
 // 5.7 us (7.4), 415,232 rows in FP32 10.0 us (12.0).
-
-// fac[dbase + n + i] = 1 / u_ii (read by the backward sweep)
-template <class T>
-__global__ void kInvDiag(int n, T *fac, int dbase) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    fac[dbase + n + i] = (T)1 / fac[dbase + i];
-}
 
 // Calls f with the largest v of the wavefront (at most W) as a compile-time
 // constant: the level loops skip the entries no row of the block has, with the

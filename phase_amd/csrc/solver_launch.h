@@ -105,12 +105,15 @@ void launchLU(phase_hip_solver *s, const IluDev<T> &L, const Scalars *sc, const 
 }
 
 template <class T>
-void launchFactor(phase_hip_solver *s, const IluDev<T> &L) {
+void factorize(phase_hip_solver *s, DBuf<T> &fac) {
+  const IluDev<T> L = iluDev<T>(s, fac.p);
   const std::vector<int> &cp = s->ord.colourPtr;
+  const size_t lds = (size_t)s->facSlots * 64 * sizeof(T);
   for (int c = 0; c + 1 < (int)cp.size(); ++c)
     if (cp[c + 1] > cp[c])
-      hipLaunchKernelGGL((kIluFactor<T>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L, s->dUpdPtr.p,
-                         s->dUpdSrc.p, s->dUpdDst.p, s->dErr.p, cp[c]);
+      hipLaunchKernelGGL((kIluFactor<T>), dim3(cp[c + 1] - cp[c]), dim3(64), lds, s->stream, L, s->rank, s->dVals.p,
+                         s->dFacSrc.p, s->dUpdPtr.p, s->dUpdSrc.p, s->dUpdDst.p, s->dErr.p, cp[c]);
+  PH_CHECK(hipGetLastError());
 }
 
 inline int spmvGrid(phase_hip_solver *s) { return std::max(1, (s->ord.nSlices + 3) / 4); }
@@ -143,17 +146,6 @@ inline void checkDeviceErr(phase_hip_solver *s) {
 
 // fac = [L slots | U slots | diagonal (n) | inverse diagonal (n)]
 inline size_t facSize(const phase_hip_solver *s) { return (size_t)s->ord.nLSlots + s->ord.nUSlots + 2 * (size_t)s->rank; }
-
-template <class T>
-void factorize(phase_hip_solver *s, DBuf<T> &fac) {
-  const int m = (int)(fac.n - s->rank);  // gathered entries: L, U, diagonal
-  hipLaunchKernelGGL((kGather<T>), dim3(gridFor(m, 256, kElemCap)), dim3(256), 0, s->stream, m,
-                     s->dFacSrc.p, s->dVals.p, fac.p);
-  launchFactor<T>(s, iluDev<T>(s, fac.p));
-  hipLaunchKernelGGL((kInvDiag<T>), dim3(gridFor(s->rank, 256, kElemCap)), dim3(256), 0, s->stream, s->rank, fac.p,
-                     s->ord.nLSlots + s->ord.nUSlots);
-  PH_CHECK(hipGetLastError());
-}
 
 inline void ensureFactor64(phase_hip_solver *s) {
   if (s->fac64Valid) return;

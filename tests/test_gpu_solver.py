@@ -52,6 +52,33 @@ def test_ilu_factor_bitwise(hip, oracle, tri_case):
     assert np.array_equal(fv, fac)
 
 
+@pytest.mark.parametrize("n,half,block_rows", [(1, 0, 64), (64, 1, 64), (65, 7, 64), (333, 7, 64), (333, 7, 7),
+                                               (1000, 3, 64), (257, 5, 1), (129, 2, 33)])
+def test_ilu_factor_row_widths_bitwise(hip, oracle, n, half, block_rows):
+    """Rows of up to 2 * half + 1 entries with a fifth of them missing (an
+    unsymmetric pattern, empty couplings in between): more and fewer entries,
+    and more and fewer updates of an entry, than the factor kernel reads ahead;
+    whole and part blocks.  Same update order as the oracle: equal bits."""
+    rng = np.random.default_rng(n + half)
+    rp, ci, v = [0], [], []
+    for i in range(n):
+        c = [j for j in range(max(0, i - half), min(n, i + half + 1)) if j == i or rng.random() < 0.8]
+        a = rng.standard_normal(len(c))
+        a[c.index(i)] = 2.0 * half + 4.0
+        ci += c
+        v += list(a)
+        rp.append(len(ci))
+    rp, ci, v = np.array(rp, np.int32), np.array(ci, np.int32), np.array(v)
+    s = _solver(hip, blockRows=block_rows)
+    s.set(rp, ci, v)
+    perm, frp, fci, fv = s.ilu_export()
+    A = H.permuted(H.compact_sorted(rp, ci, v), perm)
+    fac = oracle.ilu0(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    assert np.array_equal(frp, A.indptr)
+    assert np.array_equal(fci, A.indices)
+    assert np.array_equal(fv, fac)
+
+
 def test_export_roundtrip(hip, tri_case):
     rp, ci, v, b = tri_case
     s = _solver(hip)
