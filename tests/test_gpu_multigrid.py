@@ -8,6 +8,7 @@ dense last level (register and global-memory inverses) are all exercised;
 repeated solves are bit-identical."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
 from phase_amd import meshgen as G
@@ -100,6 +101,32 @@ def test_multigrid_dense_inverse(hip, sys1, fine, coarse, dense, lo, hi, pivotin
     k = np.linalg.cond(m)
     assert np.abs(inv @ m - np.eye(n)).max() <= 1e-13 * k, (n, k)
     print("dense level", n, "cond %.3g" % k, flush=True)
+
+
+@pytest.mark.parametrize("n,half,rows,coarse", [(200, 1, 64, 64), (333, 7, 64, 64), (5000, 5, 64, 8), (4099, 2, 7, 7),
+                                                (257, 3, 2, 64)])
+def test_galerkin_sums_exact(hip, n, half, rows, coarse):
+    """Coarse operators of a graph Laplacian plus 3 I with whole-number weights:
+    every sum is exact, so on the dense level, through all levels above it, the
+    matrix is symmetric, its entries are whole, each row sums to 3 times the
+    rows it stands for, and those add up to n.  Lists of one entry and of some
+    hundreds, none a multiple of the entries read together."""
+    rng = np.random.default_rng(n)
+    off = [sp.diags(-rng.integers(1, 9, n - d).astype(float), d) for d in range(1, half + 1)]
+    up = sum(off[1:], off[0])
+    A = up + up.T
+    A = (A + sp.diags(3. - np.asarray(A.sum(axis=1)).ravel())).tocsr()
+    A.sort_indices()
+    s = hip.HipSparseMatrixSolver(0, preconditioner="multigrid", solver="cg", mode="fp64", blockRows=rows,
+                                  multigridCoarseRows=coarse, multigridDenseRows=64)
+    s.set(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    b = rng.standard_normal(n)
+    s.set_rhs(b)
+    s.solve()
+    m, _ = s.multigrid_coarsest()
+    sums = m.sum(axis=1) / 3.
+    assert np.array_equal(m, m.T) and np.array_equal(m, np.rint(m))
+    assert np.array_equal(sums, np.rint(sums)) and sums.min() >= 1. and sums.sum() == n
 
 
 def test_multigrid_device_assembly_brick_aggregates(hip, oracle):
