@@ -104,7 +104,7 @@ int phase_hip_solver_destroy(phase_hip_solver *s);
  * "gmresRestart" (basis vectors per GMRES cycle, 1 to 64, 30), "mode"
  * (fp64|mixed|learned),
  * "innerTolerance" (mixed: residual reduction between FP64 refinement points, 0.1),
- * "maxOuter" (mixed: FP64 refinement passes, 100), "chunk" (iterations queued
+ * "maxOuter" (mixed: FP64 refinement passes, 100), "chunk" (most iterations queued
  * between host checks, 8), "blockRows" (rows per ILU aggregate, <= 64,
  * default 32; aggregates of one colour are packed into blocks of up to 64
  * rows), "ordering" (geometric | graph aggregates), "pattern" (exact | union),
