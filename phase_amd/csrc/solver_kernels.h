@@ -798,6 +798,15 @@ __device__ __forceinline__ void byMost(int v, F &&f) {
   }
 }
 
+// Keeps a sweep's first loads in flight together.  Left to itself the compiler
+// puts the loads of the block and lane records behind the test of `done`, whose
+// own load then is a round trip ahead of the chain: up to 0.5 us a launch (FP64,
+// forward: 3.36 against 3.00 us at 5,000 rows, 6.86 against 6.42 at 333,000).
+__device__ __forceinline__ void firstTrip(int done, const BlockInfo &B, const LaneRec &rec) {
+  asm volatile("" ::"s"(done), "s"(B.rowStart), "s"(B.lOff), "s"(B.uOff), "s"(B.nLev), "s"(B.nULev), "v"(rec.row),
+               "v"(rec.info));
+}
+
 // Forward sweep body for one block: returns y of the lane's row.  PRO selects
 // the fused Krylov prologue that forms the right-hand side on the fly:
 // kProP: p = r + beta (p - omega v);  kProS: s = r - alpha v (both stored);
@@ -1017,6 +1026,7 @@ __global__ __launch_bounds__(64) void kLSolve(IluDev<T> L, int blockBase, const 
   const int done = sc->done;
   const BlockInfo B = L.blocks[b];
   const LaneRec rec = L.lanes[(size_t)b * 64 + lane];
+  firstTrip(done, B, rec);
   if (done) return;  // queued past convergence
   const bool act = rec.row >= 0;
   T pro;
@@ -1043,6 +1053,7 @@ __global__ __launch_bounds__(64) void kUSolve(IluDev<T> L, int blockBase, const 
   const int done = sc->done;
   const BlockInfo B = L.blocks[b];
   const LaneRec rec = L.lanes[(size_t)b * 64 + lane];
+  firstTrip(done, B, rec);
   if (done) return;  // queued past convergence
   const bool act = rec.row >= 0;
   const T y0 = y[act ? rec.row : 0];
@@ -1074,6 +1085,7 @@ __global__ __launch_bounds__(64) void kLUSolve(IluDev<T> L, int blockBase, const
   const int done = sc->done;
   const BlockInfo B = L.blocks[b];
   const LaneRec rec = L.lanes[(size_t)b * 64 + lane];
+  firstTrip(done, B, rec);
   if (done) return;  // queued past convergence
   const bool act = rec.row >= 0;
   T pro;
