@@ -1343,8 +1343,7 @@ int phase_hip_solver_time_kernels(phase_hip_solver *s, int reps, double *ms, int
     // the launches of one preconditioner apply inside a solve: kUSolve and
     // kLSolve over every colour but the last, kLUSolve over the last; FP64
     // in 8..10, FP32 in 13..15
-    const std::vector<int> &cp = s->ord.colourPtr;
-    const int C = (int)cp.size() - 1;
+    const int C = s->ord.nColours;
     s->dR64.alloc(n);
     PH_CHECK(hipMemcpyAsync(s->dR64.p, s->dB.p, n * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
     auto perLaunch = [&](auto *fac, auto &K, double *o3, double *oc) {
@@ -1363,34 +1362,31 @@ int phase_hip_solver_time_kernels(phase_hip_solver *s, int reps, double *ms, int
         if (C >= 2) {
           o3[0] = timeIt([&] {
                     for (int c = C - 2; c >= 0; --c)
-                      hipLaunchKernelGGL((kUSolve<T, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L,
-                                         cp[c], noSc, (const T *)y, x, (const T *)nullptr, (T *)nullptr);
+                      launchUColour<T, W>(s, L, c, noSc, (const T *)y, x, (const T *)nullptr, (T *)nullptr);
                   }) / (C - 1);
           o3[2] = timeIt([&] {
                     for (int c = 0; c + 1 < C; ++c)
-                      hipLaunchKernelGGL((kLSolve<T, kProNone, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0,
-                                         s->stream, L, cp[c], noSc, in, y, (T *)nullptr, (const T *)nullptr,
-                                         (const T *)nullptr, (double *)nullptr);
+                      launchLColour<T, kProNone, W>(s, L, c, noSc, in, y, (T *)nullptr, (const T *)nullptr,
+                                                    (const T *)nullptr, (double *)nullptr);
                   }) / (C - 1);
         }
         if (C >= 1)
           o3[1] = timeIt([&] {
-            hipLaunchKernelGGL((kLUSolve<T, kProNone, W>), dim3(cp[C] - cp[C - 1]), dim3(64), 0, s->stream, L,
-                               cp[C - 1], noSc, in, (const T *)y, (T *)nullptr, (const T *)nullptr,
-                               (const T *)nullptr, x, (double *)nullptr, (const T *)nullptr, (T *)nullptr);
+            launchLUColour<T, kProNone, W>(s, L, C - 1, noSc, in, (const T *)y, (T *)nullptr, (const T *)nullptr,
+                                           (const T *)nullptr, x, (double *)nullptr, (const T *)nullptr,
+                                           (T *)nullptr);
           });
         if (C >= 2)
           oc[0] = timeIt([&] {
                     for (int c = 0; c + 1 < C; ++c)
-                      hipLaunchKernelGGL((kLSolve<T, kProCgR, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0,
-                                         s->stream, L, cp[c], noSc, (const T *)K.p.p, y, K.r.p, (const T *)nullptr,
-                                         (const T *)K.v.p, s->dR64.p);
+                      launchLColour<T, kProCgR, W>(s, L, c, noSc, (const T *)K.p.p, y, K.r.p, (const T *)nullptr,
+                                                   (const T *)K.v.p, s->dR64.p);
                   }) / (C - 1);
         if (C >= 1)
           oc[1] = timeIt([&] {
-            hipLaunchKernelGGL((kLUSolve<T, kProCgR, W>), dim3(cp[C] - cp[C - 1]), dim3(64), 0, s->stream, L,
-                               cp[C - 1], noSc, (const T *)K.p.p, (const T *)y, K.r.p, (const T *)nullptr,
-                               (const T *)K.v.p, x, s->dR64.p, (const T *)nullptr, (T *)nullptr);
+            launchLUColour<T, kProCgR, W>(s, L, C - 1, noSc, (const T *)K.p.p, (const T *)y, K.r.p,
+                                          (const T *)nullptr, (const T *)K.v.p, x, s->dR64.p, (const T *)nullptr,
+                                          (T *)nullptr);
           });
       });
     };

@@ -915,7 +915,8 @@ __device__ __forceinline__ T lBody(const IluDev<T> &L, const BlockInfo &B, bool 
 
 // Backward sweep of one block in two parts: uLoad issues every load the row
 // needs from the factor, uSolve gathers later-coloured solution values and
-// runs the levels from acc = y of the lane's row, returning x of the row.
+// runs the levels from acc = y of the lane's row, returning x of the row; REG:
+// out of registers (else through the LDS array: the same sums, same bits).
 // In-block columns precede later-block columns, as in the oracle's back
 // substitution.
 template <class T, int W>
@@ -960,7 +961,7 @@ __device__ __forceinline__ void uLoad(const IluDev<T> &L, const BlockInfo &B, bo
   }
 }
 
-template <class T, int W>
+template <class T, int W, bool REG>
 __device__ __forceinline__ T uSolve(const IluDev<T> &L, const BlockInfo &B, bool act, int lane, T acc,
                                     const T *__restrict__ x, T *xlds, const UPre<T, W> &u) {
   asm volatile("" ::: "memory");
@@ -982,15 +983,17 @@ __device__ __forceinline__ T uSolve(const IluDev<T> &L, const BlockInfo &B, bool
       soff = fma(facU[s], x[L.uCol[s]], soff);
     }
   }
-  if (W == 8 && __any(u.nIn > W)) {
+  if (!REG || (W == 8 && __any(u.nIn > W))) {
     for (int l = 0; l < B.nULev; ++l) {
       if (act && u.ulev == l) {
 #pragma unroll
         for (int q = 0; q < W; ++q)
           if (q < u.nIn) acc = fma(-u.uv[q], xlds[u.uc[q] - B.rowStart], acc);
-        for (int e = W; e < u.nIn; ++e) {
-          const int s = B.uOff + (e << 6) + lane;
-          acc = fma(-facU[s], xlds[L.uCol[s] - B.rowStart], acc);
+        if constexpr (W == 8) {
+          for (int e = W; e < u.nIn; ++e) {
+            const int s = B.uOff + (e << 6) + lane;
+            acc = fma(-facU[s], xlds[L.uCol[s] - B.rowStart], acc);
+          }
         }
         acc = (acc - soff) * u.d;
         xlds[lane] = acc;
@@ -1043,7 +1046,7 @@ __global__ __launch_bounds__(64) void kLSolve(IluDev<T> L, int blockBase, const 
 // the finished x of each row is also added to addFrom's value into addTo
 // (z = z + M^-1 t of a multigrid post-smoothing, without a launch of its own;
 // addFrom may be addTo).
-template <class T, int W = 8>
+template <class T, int W = 8, bool REG = true>
 __global__ __launch_bounds__(64) void kUSolve(IluDev<T> L, int blockBase, const Scalars *sc,
                                               const T *__restrict__ y, T *__restrict__ x,
                                               const T *addFrom, T *addTo) {
@@ -1059,7 +1062,7 @@ __global__ __launch_bounds__(64) void kUSolve(IluDev<T> L, int blockBase, const 
   const T y0 = y[act ? rec.row : 0];
   UPre<T, W> u;
   uLoad<T, W>(L, B, act, rec.row, rec.info, lane, u);
-  const T acc = uSolve<T, W>(L, B, act, lane, act ? y0 : (T)0, x, xlds, u);
+  const T acc = uSolve<T, W, REG>(L, B, act, lane, act ? y0 : (T)0, x, xlds, u);
   if (act) {
     x[rec.row] = acc;
     if (addTo) addTo[rec.row] = addFrom[rec.row] + acc;
@@ -1072,7 +1075,7 @@ __global__ __launch_bounds__(64) void kUSolve(IluDev<T> L, int blockBase, const 
 // entries load after the forward levels: issued up front they overlap the
 // forward sweep's loads but double the registers, and the lower occupancy
 // costs more (a second round of blocks per launch) than the round trip.
-template <class T, int PRO, int W = 8>
+template <class T, int PRO, int W = 8, bool REG = true>
 __global__ __launch_bounds__(64) void kLUSolve(IluDev<T> L, int blockBase, const Scalars *sc,
                                                const T *__restrict__ in, const T *__restrict__ y,
                                                T *__restrict__ pv, const T *__restrict__ r,
@@ -1093,7 +1096,7 @@ __global__ __launch_bounds__(64) void kLUSolve(IluDev<T> L, int blockBase, const
   const T yv = lBody<T, PRO, W>(L, B, act, rec.row, rec.info, lane, sc, in, y, pv, r, v, ylds, pro, xs, xo);
   UPre<T, W> u;
   uLoad<T, W>(L, B, act, rec.row, rec.info, lane, u);
-  const T acc = uSolve<T, W>(L, B, act, lane, yv, x, xlds, u);
+  const T acc = uSolve<T, W, REG>(L, B, act, lane, yv, x, xlds, u);
   if (act) {
     if (PRO != kProNone) pv[rec.row] = pro;
     if (PRO == kProCgR) xs[rec.row] = xo;

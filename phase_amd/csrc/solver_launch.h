@@ -52,6 +52,63 @@ void byWidth(const phase_hip_solver *s, F &&f) {
   else f(std::integral_constant<int, 8>());
 }
 
+// Calls f with the backward levels' form for a launch of `blocks` blocks (fused:
+// kLUSolve) as a compile-time constant: out of registers, or through the LDS
+// array.  An FP64 value is two crossbar words, which the register form moves for
+// every lane at every level, the array only for the level's rows.  Once the
+// launch fills the chip the crossbar counts, not the trip: of kLUSolve from some
+// 4,000 blocks (15 wavefronts a CU) on -- 3,000 blocks of quads 5.80 us in
+// registers, 6.48 through the array; 3,900 of triangles 8.18 and 7.90; 6,500
+// 11.47 and 10.49; 19,500 24.59 and 22.77 --, of kUSolve, whose blocks are
+// shorter, only while one generation of wavefronts (32 on each of 256 CUs) holds
+// the whole launch: 4,500 blocks 6.74 and 6.68, 5,500 7.84 and 7.40, 6,500 8.58
+// and 8.03, but 8,600 10.16 and 10.21, 15,000 of quads 12.05 and 12.99.  FP32
+// moves one word: in registers always.  (The forward levels too: 6.35 us against
+// 6.65 at 6,500 blocks in FP64.)
+constexpr int kLdsFusedBlocks = 4096, kLdsBlocks = 5120, kOneGeneration = 32 * 256;
+inline bool backwardInRegisters(bool fp64, bool fused, int blocks) {
+  if (!fp64) return true;
+  return fused ? blocks <= kLdsFusedBlocks : blocks <= kLdsBlocks || blocks > kOneGeneration;
+}
+template <class T, class F>
+void byLevels(bool fused, int blocks, F &&f) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (!backwardInRegisters(true, fused, blocks)) return f(std::false_type());
+  }
+  f(std::true_type());
+}
+
+// One colour's sweep launch each.
+template <class T, int PRO, int W>
+void launchLColour(phase_hip_solver *s, const IluDev<T> &L, int c, const Scalars *sc, const T *in, T *y, T *pv,
+                   const T *r, const T *v, double *xs) {
+  const int first = s->ord.colourPtr[c], blocks = s->ord.colourPtr[c + 1] - first;
+  if (blocks < 1) return;
+  hipLaunchKernelGGL((kLSolve<T, PRO, W>), dim3(blocks), dim3(64), 0, s->stream, L, first, sc, in, y, pv, r, v, xs);
+}
+
+template <class T, int W>
+void launchUColour(phase_hip_solver *s, const IluDev<T> &L, int c, const Scalars *sc, const T *y, T *x,
+                   const T *addFrom, T *addTo) {
+  const int first = s->ord.colourPtr[c], blocks = s->ord.colourPtr[c + 1] - first;
+  if (blocks < 1) return;
+  byLevels<T>(false, blocks, [&](auto reg) {
+    hipLaunchKernelGGL((kUSolve<T, W, decltype(reg)::value>), dim3(blocks), dim3(64), 0, s->stream, L, first, sc, y, x,
+                       addFrom, addTo);
+  });
+}
+
+template <class T, int PRO, int W>
+void launchLUColour(phase_hip_solver *s, const IluDev<T> &L, int c, const Scalars *sc, const T *in, const T *y, T *pv,
+                    const T *r, const T *v, T *out, double *xs, const T *addFrom, T *addTo) {
+  const int first = s->ord.colourPtr[c], blocks = s->ord.colourPtr[c + 1] - first;
+  if (blocks < 1) return;
+  byLevels<T>(true, blocks, [&](auto reg) {
+    hipLaunchKernelGGL((kLUSolve<T, PRO, W, decltype(reg)::value>), dim3(blocks), dim3(64), 0, s->stream, L, first, sc,
+                       in, y, pv, r, v, out, xs, addFrom, addTo);
+  });
+}
+
 // Sweep launchers: one launch per block colour (forward colours ascending,
 // backward descending).
 template <class T, int PRO>
@@ -59,11 +116,7 @@ void launchL(phase_hip_solver *s, const IluDev<T> &L, const Scalars *sc, const T
              const T *v, double *xs = nullptr) {
   byWidth(s, [&](auto Wc) {
     constexpr int W = decltype(Wc)::value;
-    const std::vector<int> &cp = s->ord.colourPtr;
-    for (int c = 0; c + 1 < (int)cp.size(); ++c)
-      if (cp[c + 1] > cp[c])
-        hipLaunchKernelGGL((kLSolve<T, PRO, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L, cp[c], sc, in,
-                           y, pv, r, v, xs);
+    for (int c = 0; c < s->ord.nColours; ++c) launchLColour<T, PRO, W>(s, L, c, sc, in, y, pv, r, v, xs);
   });
 }
 
@@ -71,11 +124,8 @@ template <class T>
 void launchU(phase_hip_solver *s, const IluDev<T> &L, const Scalars *sc, const T *y, T *x) {
   byWidth(s, [&](auto Wc) {
     constexpr int W = decltype(Wc)::value;
-    const std::vector<int> &cp = s->ord.colourPtr;
-    for (int c = (int)cp.size() - 2; c >= 0; --c)
-      if (cp[c + 1] > cp[c])
-        hipLaunchKernelGGL((kUSolve<T, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L, cp[c], sc, y, x,
-                           (const T *)nullptr, (T *)nullptr);
+    for (int c = s->ord.nColours - 1; c >= 0; --c)
+      launchUColour<T, W>(s, L, c, sc, y, x, (const T *)nullptr, (T *)nullptr);
   });
 }
 
@@ -85,22 +135,13 @@ void launchU(phase_hip_solver *s, const IluDev<T> &L, const Scalars *sc, const T
 template <class T, int PRO>
 void launchLU(phase_hip_solver *s, const IluDev<T> &L, const Scalars *sc, const T *in, T *y, T *pv, const T *r,
               const T *v, T *out, double *xs = nullptr, const T *addFrom = nullptr, T *addTo = nullptr) {
-  const std::vector<int> &cp = s->ord.colourPtr;
-  const int C = (int)cp.size() - 1;
+  const int C = s->ord.nColours;
   if (C < 1) return;
   byWidth(s, [&](auto Wc) {
     constexpr int W = decltype(Wc)::value;
-    for (int c = 0; c + 1 < C; ++c)
-      if (cp[c + 1] > cp[c])
-        hipLaunchKernelGGL((kLSolve<T, PRO, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L, cp[c], sc, in,
-                           y, pv, r, v, xs);
-    if (cp[C] > cp[C - 1])
-      hipLaunchKernelGGL((kLUSolve<T, PRO, W>), dim3(cp[C] - cp[C - 1]), dim3(64), 0, s->stream, L, cp[C - 1], sc,
-                         in, (const T *)y, pv, r, v, out, xs, addFrom, addTo);
-    for (int c = C - 2; c >= 0; --c)
-      if (cp[c + 1] > cp[c])
-        hipLaunchKernelGGL((kUSolve<T, W>), dim3(cp[c + 1] - cp[c]), dim3(64), 0, s->stream, L, cp[c], sc,
-                           (const T *)y, out, addFrom, addTo);
+    for (int c = 0; c + 1 < C; ++c) launchLColour<T, PRO, W>(s, L, c, sc, in, y, pv, r, v, xs);
+    launchLUColour<T, PRO, W>(s, L, C - 1, sc, in, y, pv, r, v, out, xs, addFrom, addTo);
+    for (int c = C - 2; c >= 0; --c) launchUColour<T, W>(s, L, c, sc, y, out, addFrom, addTo);
   });
 }
 

@@ -7,6 +7,7 @@ agreement with a direct (scipy splu) solution within cond-scaled bounds.
 """
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
 from tests import helpers as H
@@ -77,6 +78,35 @@ def test_ilu_factor_row_widths_bitwise(hip, oracle, n, half, block_rows):
     assert np.array_equal(frp, A.indptr)
     assert np.array_equal(fci, A.indices)
     assert np.array_equal(fv, fac)
+
+
+@pytest.mark.parametrize("per_colour,half", [(4096, 3), (4097, 3), (4097, 5), (5120, 3), (5121, 3), (5121, 5),
+                                             (8192, 3), (8193, 3)])
+def test_sweep_forms_by_blocks(hip, per_colour, half):
+    """The sweeps' backward levels change their form with the blocks of a launch
+    (FP64: fused above 4,096, the other colour between 5,121 and 8,192).  One
+    GMRES step from zero leaves x = alpha M^-1 b: every row of L U x must be alpha
+    b to the round-off of two substitutions, gamma_k |L||U||x| with k the rows'
+    entries (at most 6 and 6) and a few roundings of the step's scalings."""
+    rows = 33  # more than half a block: one aggregate per block
+    n = 2 * per_colour * rows
+    rng = np.random.default_rng(per_colour)
+    offs = range(-half, half + 1)
+    A = sp.diags([rng.uniform(-1.0, 1.0, n - abs(d)) + (12.0 if d == 0 else 0.0) for d in offs], offs).tocsr()
+    b = rng.standard_normal(n)
+    s = _solver(hip, solver="gmres", blockRows=rows, maxIters=1, tolerance=1e-14)
+    s.set(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    s.set_rhs(b)
+    o = s.ordering_info()
+    assert o == {"blocks": 2 * per_colour, "colours": 2}
+    s.solve(raise_on_noconv=False)
+    perm, rp, ci, v = s.ilu_export()
+    x, r = s.x()[perm], b[perm]
+    F = sp.csr_matrix((v, ci, rp), shape=(n, n))
+    L, U = sp.tril(F, -1).tocsr() + sp.identity(n, format="csr"), sp.triu(F).tocsr()
+    lux = L @ (U @ x)
+    alpha = (lux @ r) / (r @ r)
+    assert np.all(np.abs(lux - alpha * r) <= 32 * 2.0 ** -53 * (abs(L) @ (abs(U) @ np.abs(x)) + np.abs(alpha * r)))
 
 
 def test_export_roundtrip(hip, tri_case):
