@@ -50,11 +50,15 @@ constexpr int kGmGroup = 8;
 constexpr double kGmMixedDrop = 1e-5;  // a mixed cycle's reduction of the residual estimate
 constexpr int kGmMixedStall = 3;
 
-// Blocks of the dot products, at most: one per CU.  A block's sums of kGmGroup
-// vectors cost it as much as several rows a thread, and every kGmAxpy block
-// reads the partials (at 200,000 rows one row a thread, 782 blocks, took
-// 13.2 us); up to 65,536 rows a row a thread keeps more CUs busy.
-constexpr int kGmDotBlocks = 256;
+// Blocks of the dot products, at most.  A block's sums of kGmGroup vectors cost
+// it as much as several rows a thread, and every kGmAxpy block reads the
+// partials: up to 65,536 rows a row a thread, up to 262,144 one block per CU (at
+// 200,000 rows a row a thread, 782 blocks, took 13.2 us a launch, 256 blocks
+// 10.8).  A larger basis needs more wavefronts in flight than that leaves: two
+// blocks per CU up to 2^20 rows, then four.  A step of 30 vectors, FP64 cycles
+// with ILU(0): 400,000 rows 115 us with one block per CU, 105 with two (four:
+// 114); one million 217, 188 (192); two million 431, 351 (340).
+inline int dotBlocks(int n) { return gridFor(n, kRedBlock, n <= 1 << 18 ? 256 : n <= 1 << 20 ? 512 : 1024); }
 
 // partials of (w, V_j) for the kGmGroup vectors j = 8 blockIdx.y + q < k
 template <class T>
@@ -88,12 +92,14 @@ __global__ __launch_bounds__(kRedBlock) void kGmAxpy(int n, int k, const T *__re
   __shared__ double h[kGmMaxRestart + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int j = wave; j < k; j += kRedBlock / 64) {
-    double t[kGmDotBlocks / 64], acc = 0.;
+    double acc = 0.;
+    for (int b0 = lane; b0 < lane + G; b0 += 256) {
+      double t[4];
 #pragma unroll
-    for (int u = 0; u < kGmDotBlocks / 64; ++u)
-      t[u] = lane + 64 * u < G ? dotPart[(size_t)j * G + lane + 64 * u] : 0.;
+      for (int u = 0; u < 4; ++u) t[u] = b0 + 64 * u < G ? dotPart[(size_t)j * G + b0 + 64 * u] : 0.;
 #pragma unroll
-    for (int u = 0; u < kGmDotBlocks / 64; ++u) acc += t[u];
+      for (int u = 0; u < 4; ++u) acc += t[u];
+    }
     acc = waveSum(acc);
     if (lane == 0) {
       h[j] = acc;
@@ -262,7 +268,7 @@ int gmresCycles(phase_hip_solver *s, double b2, int budget, bool *stalled) {
   hipStream_t st = s->stream;
   const IluDev<T> L = iluDev<T>(s, factor<T>(s));
   const int G = gridFor(n, kRedBlock, kRedCap);
-  const int Gd = gridFor(n, kRedBlock, kGmDotBlocks), Ga = gridFor(n, kRedBlock, 2 * kGmDotBlocks);
+  const int Gd = dotBlocks(n), Ga = gridFor(n, kRedBlock, std::min(2 * Gd, kRedCap));
   const int groups = (m + 1 + kGmGroup - 1) / kGmGroup;
   gmBasis<T>(s).alloc((size_t)(m + 1) * n);
   gmPrec<T>(s).alloc((size_t)m * n);

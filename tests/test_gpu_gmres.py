@@ -10,6 +10,7 @@ restarted from the FP64 residual) reaches the same FP64 goal, and continues
 in FP64 when its FP32 cycles cannot run."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
 from tests import helpers as H
@@ -51,6 +52,34 @@ def test_gmres_matches_direct(hip, sys1, prec, restart, mode):
     assert true <= 1.5e-8 and abs(true - rel) <= 1e-3 * rel + 1e-14
     assert np.linalg.norm(x - x_ref) <= kappa * 1.5e-8 * np.linalg.norm(x_ref)
     print(prec, restart, mode, "iterations", s.n_iters(), flush=True)
+
+
+@pytest.mark.parametrize("n", [65537, 131073, 262144, 262145, 1 << 20, (1 << 20) + 1, 1100003])
+def test_gmres_large_bases(hip, n):
+    """Above 65,536 rows a thread of the basis' dot products takes several rows,
+    above 262,144 and 2^20 with more blocks.  On a diagonally dominant band
+    (|x| <= 2 |A x|: each row's diagonal exceeds its other entries by at least 0.5)
+    one cycle reaches the goal; a wrong dot product or update leaves the basis
+    not orthogonal, and the cycle's own residual away from the true one, which
+    would take another cycle."""
+    rng = np.random.default_rng(n)
+    offs = [d for d in range(-3, 4) if d]
+    A = sp.diags([rng.uniform(-1.0, 1.0, n - abs(d)) for d in offs], offs).tocsr()
+    A = (A + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel() + 0.5)).tocsr()
+    x_ref = rng.standard_normal(n)
+    b = A @ x_ref
+    rp, ci = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+    for mode, tol in (("fp64", 1e-8), ("mixed", 1e-5)):
+        s = hip.HipSparseMatrixSolver(0, tolerance=tol, maxIters=200, solver="gmres", mode=mode)
+        s.set(rp, ci, A.data)
+        s.set_rhs(b)
+        rel = s.solve()
+        x = s.x()
+        true = np.linalg.norm(b - A @ x) / np.linalg.norm(b)
+        assert rel <= tol and abs(true - rel) <= 1e-3 * rel
+        assert s.stats()["outer_passes"] == 2, s.stats()
+        assert np.abs(x - x_ref).max() <= 2 * np.abs(b - A @ x).max() + 1e-15 * np.abs(x_ref).max()
+        print(n, mode, s.n_iters(), rel, flush=True)
 
 
 def test_mixed_gmres_continues_in_fp64(hip, sys1):
