@@ -917,7 +917,14 @@ __global__ __launch_bounds__(kRedBlock) void kMlJacDirection(int n, int nSlices,
 // and 540 rows 8.9 us a V cycle (FP64; five launches 21 us).
 constexpr int kTailBlock = 1024;
 constexpr int kTailInvBytes = 104 * 1024;  // LDS for block inverses, beside at most 52 KB of vectors
-constexpr int kTailRows = 4;  // rows per thread at most: 64 registers of matrix values
+// Rows per thread and dense rows at most.  A fourth row's matrix entries spill
+// (128 to 236 B a lane; three rows 0 to 64), and past 256 dense rows one CU reads
+// the inverse for longer than the launches it saves; an iteration of a solve with
+// the level as launches / in one workgroup: 2,825 rows over 203 dense ones 143 /
+// 127 us (K cycle, FP64; FP32 134 / 116, V cycles 104 / 106 and 100 / 100), 3,087 over 215
+// 141 / 153 (FP32 134 / 131, V cycles 105 / 116 and 101 / 108), 4,084 over 292 148 / 169
+// (137 / 149, 108 / 127, 102 / 121), but 2,825 over 399 142 / 152 (V cycle 104 / 114).
+constexpr int kTailRows = 3, kTailDense = 256;
 // Entries of a row in registers: rows of brick aggregates have about 7, of graph
 // aggregates up to 14 and more.
 constexpr int tailWidth(int rows) { return rows == 1 ? 16 : rows == 2 ? 12 : 8; }
@@ -940,10 +947,10 @@ __global__ __launch_bounds__(kTailBlock) void kMlTail(TailLevel<T> L, const T *_
   constexpr int W = tailWidth(R);
   __shared__ T xs[kTailBlock * R];                               // what the products gather from
   __shared__ T z1s[KCYCLE ? kTailBlock * R : 1], q1s[KCYCLE ? kTailBlock * R : 1];
-  __shared__ T rc[kDenseMax], ec[kDenseMax];
+  __shared__ T rc[kTailDense], ec[kTailDense];
   __shared__ __align__(16) double part[2 * kTailBlock];
   __shared__ double red[2][kTailBlock / 64];
-  __shared__ int ap[kDenseMax + 1];
+  __shared__ int ap[kTailDense + 1];
   // the block inverses, where they fit (one row a thread): a K cycle applies
   // them four times, and out of L2 each costs three round trips
   constexpr int kInvLds = ILU && R == 1 ? kTailInvBytes / (int)sizeof(T) : 1;
@@ -1243,14 +1250,16 @@ template <class T>
 void cycle(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, const T *r, T *e);
 
 // Level l and the dense level below it run as one workgroup (kMlTail): no more
-// rows than its threads hold in registers, and with ILU(0) smoothing
+// rows than its threads hold in registers over at most kTailDense dense ones, and with ILU(0) smoothing
 // block-diagonal in the aggregates and at most kTailIluRows, whose block
-// inverses (some 20 entries a row) are read from L2 at every smoothing.  A
-// larger level keeps its launches, whose blocks then share the work.
+// inverses (some 20 entries a row) are read from L2 at every smoothing (an
+// iteration as launches / in one workgroup at 1,062 rows: BiCGStab 212 / 202 us in
+// FP64, 207 / 177 mixed, GMRES 193 / 143; at 1,785 220 / 199, 211 / 185, 192 / 144).
+// A larger level keeps its launches, whose blocks then share the work.
 constexpr int kTailIluRows = 2 * kTailBlock;
 bool tailLevel(const Multilevel &M, int l) {
   const MlLevel &L = M.lv[l];
-  if (!L.sol || M.lv[l + 1].sol) return false;
+  if (!L.sol || M.lv[l + 1].sol || M.lv[l + 1].n > kTailDense) return false;
   return L.jacobi ? L.n <= kTailBlock * kTailRows : L.blockWidth > 0;
 }
 
@@ -1278,8 +1287,7 @@ void launchTail(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, co
   }
   if (rows <= 1) go(std::integral_constant<int, 1>());
   else if (rows == 2) go(std::integral_constant<int, 2>());
-  else if (rows == 3) go(std::integral_constant<int, 3>());
-  else go(std::integral_constant<int, 4>());
+  else go(std::integral_constant<int, 3>());
 }
 
 // e = (approximate) A_l^-1 r at coarse level l

@@ -205,12 +205,15 @@ def test_multigrid_graph_aggregates_wide_coarse_rows(hip, oracle):
 
 
 @pytest.mark.parametrize("cycle", ["K", "V"])
-@pytest.mark.parametrize("nx,rows", [(128, 1), (170, 1), (180, 2), (250, 3), (350, 4), (360, 5)])
-def test_last_levels_match_direct(hip, oracle, nx, rows, cycle):
-    """The level above the dense one in one workgroup, at 1 to 4 rows per thread
-    (565 to 4,084 rows, 979 and 1,100 and 4,084 at the edges; graph aggregates,
+@pytest.mark.parametrize("nx,rows,coarse", [(128, 1, 16), (170, 1, 16), (180, 2, 16), (250, 3, 16), (300, 3, 16),
+                                            (303, 4, 16), (350, 4, 16), (360, 5, 16), (170, 1, 4), (230, 2, 8),
+                                            (250, 3, 6)])
+def test_last_levels_match_direct(hip, oracle, nx, rows, coarse, cycle):
+    """The level above the dense one in one workgroup, at 1 to 3 rows per thread
+    (565 to about 3,000 rows, 979 and 1,100 at the edges; graph aggregates,
     whose rows are partly wider than the entries held in registers), and as
-    launches above that (4,316 rows).  A solve to 1e-10 is within
+    launches above that (3,087 to 4,316 rows) and over more than 256 dense rows
+    (2,110 over 370; 979 over 254 and 1,785 over 237 below the line).  A solve to 1e-10 is within
     cond(A) 1e-10 of the direct one; cond(A) is below 16 nx^2 for these
     coefficients (8 / pi^2 nx^2 times the spread e^(4 sigma) within four
     deviations, sigma = 0.5).  A wrong coarse correction shows in the iteration
@@ -220,7 +223,8 @@ def test_last_levels_match_direct(hip, oracle, nx, rows, cycle):
     x_ref = spla.splu(A.tocsc()).solve(b)
     for mode in ("fp64", "mixed"):
         s = hip.HipSparseMatrixSolver(0, tolerance=1e-10, maxIters=2000, solver="cg", mode=mode,
-                                      preconditioner="multigrid", multigridDenseRows=512, multigridCycle=cycle)
+                                      preconditioner="multigrid", multigridDenseRows=512, multigridCycle=cycle,
+                                      multigridCoarseRows=coarse)
         s.set(rp, ci, v)
         s.set_rhs(b)
         s.solve()
