@@ -21,6 +21,10 @@ struct MlScalars {
   double pq1, alpha1, gamma, alpha2;
 };
 
+// Most rows of a finest level whose prolongation and post-smoothing residual run
+// as one launch (smoothCorrectSmooth).
+constexpr int kFusedProlongRows = 1 << 18;
+
 template <class T>
 struct MlVecs {
   // r: right-hand side, e: solution of this level's coarse solve; t, w, y, u:
@@ -29,9 +33,11 @@ struct MlVecs {
   void alloc(int n) {
     for (DBuf<T> *b : {&r, &e, &t, &w, &y, &u, &z1, &q1, &r1, &z2}) b->alloc(n);
   }
-  // the finest level uses the cycle work vectors only
+  // the finest level uses the cycle work vectors only, u where its prolongation
+  // runs with the post-smoothing residual
   void allocCycle(int n) {
-    for (DBuf<T> *b : {&t, &w, &y, &u}) b->alloc(n);
+    for (DBuf<T> *b : {&t, &w, &y}) b->alloc(n);
+    if (n <= kFusedProlongRows) u.alloc(n);
   }
 };
 
@@ -1366,7 +1372,6 @@ void coarseSolve(phase_hip_solver *s, Multilevel &M, int l, const Scalars *sc, c
 // at 16,384 rows, 7.6 against 8.7 at 200,000, 20.5 against 18.1 at one million): the line
 // is drawn at kFusedProlongRows.  The post-smoothing sweep adds its result into z
 // as it finishes each row.  The arithmetic is that of the separate kernels.
-constexpr int kFusedProlongRows = 1 << 18;
 template <class T>
 void smoothCorrectSmooth(phase_hip_solver *s, Multilevel &M, phase_hip_solver *c, MlVecs<T> &V, int next,
                          const Scalars *sc, const T *r, T *z, bool pre, bool post = true) {

@@ -6,6 +6,8 @@ preconditioner cuts the iteration count against ILU(0) alone; K and V cycles,
 damped-Jacobi and ILU(0) smoothing of the coarse levels, nested levels and the
 dense last level (register and global-memory inverses) are all exercised;
 repeated solves are bit-identical."""
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -236,6 +238,36 @@ def test_last_levels_match_direct(hip, oracle, nx, rows, coarse, cycle):
         s.zero_guess()
         s.solve()
         assert np.array_equal(s.x(), x)
+
+
+@pytest.mark.parametrize("mode,most", [("fp64", 208), ("mixed", 242)])
+def test_multigrid_memory(hip, mode, most):
+    """Device memory a first multigrid solve of 2^19 rows takes: Krylov and cycle
+    vectors, factors and hierarchy, 204 bytes a row in FP64 and 236 mixed (in
+    whole 2 MB; the rows' five entries are set before).  A vector that nothing
+    reads would be 8 bytes more, 12 in mixed mode."""
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.load_library().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    def solver(n):
+        off = [sp.diags(-np.ones(n - d), d) for d in (1, 2)]
+        up = off[0] + off[1]
+        A = up + up.T
+        A = (A + sp.diags(3. - np.asarray(A.sum(axis=1)).ravel())).tocsr()
+        s = hip.HipSparseMatrixSolver(0, solver="cg", mode=mode, preconditioner="multigrid", maxIters=3)
+        s.set(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+        s.set_rhs(np.ones(n))
+        return s
+
+    solver(5000).solve(raise_on_noconv=False)  # the kernels are loaded
+    n = 1 << 19
+    s = solver(n)
+    before = free()
+    s.solve(raise_on_noconv=False)
+    taken = before - free()
+    assert taken <= most * n, taken / n
 
 
 @pytest.mark.parametrize("solver", ["bicgstab", "gmres"])
