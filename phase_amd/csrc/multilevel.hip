@@ -1567,7 +1567,8 @@ void mlEnsureHierarchy(phase_hip_solver *s) {
         // can the ILU(0) level above run as kMlTail: its blocks are the aggregates
         if (level > 0) {
           MlLevel &U = M->lv[level - 1];
-          if (!U.jacobi && U.sol->blockJacobi && U.n <= kTailIluRows && (int)fine->blocks.size() == c.n) {
+          if (!U.jacobi && U.sol->blockJacobi && U.n <= kTailIluRows && c.n <= kTailDense &&
+              (int)fine->blocks.size() == c.n) {
             int width = 0;
             for (int a = 0; a < c.n; ++a) {
               const BlockInfo &B = fine->blocks[a];
@@ -1654,14 +1655,12 @@ void mlEnsureValues(phase_hip_solver *s, bool single) {
           L.dinv32.alloc(L.n);
           hipLaunchKernelGGL((kConvert<double, float>), dim3(elemGrid(L.n)), dim3(256), 0, st, L.n, L.dinv64.p,
                              L.dinv32.p);
+        } else if (L.blockWidth > 0) {  // kMlTail: the blocks' inverses, no factor
+          const int m = (int)L.binv64.n;
+          L.binv32.alloc(m);
+          hipLaunchKernelGGL((kConvert<double, float>), dim3(elemGrid(m)), dim3(256), 0, st, m, L.binv64.p, L.binv32.p);
         } else if (L.sol) {
           ensureSingle(L.sol);
-          if (L.blockWidth > 0) {
-            const int m = (int)L.binv64.n;
-            L.binv32.alloc(m);
-            hipLaunchKernelGGL((kConvert<double, float>), dim3(elemGrid(m)), dim3(256), 0, st, m, L.binv64.p,
-                               L.binv32.p);
-          }
         }
       M.singleValid = true;
     }

@@ -271,23 +271,24 @@ def test_multigrid_memory(hip, mode, most):
 
 
 @pytest.mark.parametrize("solver", ["bicgstab", "gmres"])
-@pytest.mark.parametrize("nx,rows", [(128, 1), (170, 1), (180, 2), (250, 3)])
-def test_last_levels_ilu_match_direct(hip, oracle, nx, rows, solver):
+@pytest.mark.parametrize("nx,rows,coarse,lo,hi", [(128, 1, 16, 1, 256), (170, 1, 16, 1, 256), (180, 2, 16, 1, 256),
+                                                  (250, 3, 16, 1, 256), (230, 2, 4, 257, 512)])
+def test_last_levels_ilu_match_direct(hip, oracle, nx, rows, coarse, lo, hi, solver):
     """As above with ILU(0)-smoothed coarse levels: V cycles under BiCGStab, K
     cycles under GMRES; 565 to 1,100 rows in one workgroup (block inverses),
-    2,110 as launches."""
+    2,110 as launches, and 1,785 over more than 256 dense rows."""
     m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, nx), sigma=0.5)
     A = H.compact_sorted(rp, ci, v)
     x_ref = spla.splu(A.tocsc()).solve(b)
     for mode in ("fp64", "mixed"):
         s = hip.HipSparseMatrixSolver(0, tolerance=1e-10, maxIters=2000, solver=solver, mode=mode,
-                                      preconditioner="multigrid")
+                                      preconditioner="multigrid", multigridCoarseRows=coarse, multigridDenseRows=hi)
         s.set(rp, ci, v)
         s.set_rhs(b)
         s.solve()
         x = s.x()
         lv = s.multigrid_levels()
-        assert (lv[1] + 1023) // 1024 == rows, lv
+        assert (lv[1] + 1023) // 1024 == rows and lo <= lv[2] <= hi, lv
         assert np.linalg.norm(x - x_ref) <= 16 * nx * nx * 1e-10 * np.linalg.norm(x_ref)
         assert s.n_iters() <= 200
         s.zero_guess()
