@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -166,6 +168,19 @@ struct Scalars {
   double minRatio;        // learned mode: smallest accepted ||r_k||/||r_{k-1}|| ... (<=0 disables)
   double rhoNext;         // CG: (r, z) of the newest z, taken over as rho by the next alpha
 };
+
+// Krylov iterations to queue next, at most `chunk`: as many as the rate of
+// decrease since the last look needs to reach tol2.  rr is ||r||^2 as the device
+// holds it after `it` iterations, rrLast the same after itLast (0: the starting
+// residual).  BiCGStab forms it at an iteration's end, CG on entry to one, of the
+// residual that the iteration before left: a CG run's rr is that of it - 1, and
+// the iteration that meets the threshold is the one after.
+inline int nextChunk(double rrLast, double rr, double tol2, int itLast, int it, bool cg, int chunk) {
+  const int steps = cg ? it - 1 - std::max(itLast - 1, 0) : it - itLast;
+  if (!(rrLast > 0. && rr > tol2 && rr < rrLast && steps > 0)) return chunk;
+  const double need = std::log(tol2 / rr) / (std::log(rr / rrLast) / steps);
+  return need < chunk ? std::max(1, (int)std::ceil(need)) : chunk;
+}
 
 enum { kDoneRunning = 0, kDoneConverged = 1, kDoneBreakdown = 2, kDoneMaxIters = 3,
        kDoneStagnation = 4 };

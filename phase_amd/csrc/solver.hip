@@ -199,11 +199,7 @@ int runKrylov(phase_hip_solver *s, KrylovVecs<T> &K, DBuf<T> &fac, const TV *sel
     it = h.iters;
     if (h.done != kDoneRunning || it >= budget) break;
     if (!onChunk(it)) break;
-    chunk = s->chunk;
-    if (rrLast > 0. && h.rr > h.tol2 && h.rr < rrLast && it > itLast) {
-      const double need = std::log(h.tol2 / h.rr) / (std::log(h.rr / rrLast) / (it - itLast));
-      if (need < chunk) chunk = std::max(1, (int)std::ceil(need));
-    }
+    chunk = nextChunk(rrLast, h.rr, h.tol2, itLast, it, s->cg, s->chunk);
     rrLast = h.rr;
     itLast = it;
   }

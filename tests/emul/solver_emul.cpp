@@ -340,3 +340,8 @@ extern "C" int emul_hierarchy(int n, const int *rowPtr, const int *colInd, const
     return -1;
   }
 }
+
+// The product's rule for the Krylov iterations queued between host checks.
+extern "C" int emul_next_chunk(double rrLast, double rr, double tol2, int itLast, int it, int cg, int chunk) {
+  return nextChunk(rrLast, rr, tol2, itLast, it, cg != 0, chunk);
+}

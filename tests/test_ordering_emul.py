@@ -258,3 +258,28 @@ def test_emul_block_jacobi_ordering(oracle, emul):
     y, x = oracle.lu_solve(Ab.indptr, Ab.indices, fac, b_solver)
     assert np.array_equal(r["y"], y)
     assert np.linalg.norm(r["x"] - x) <= 1e-12 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("cg", [0, 1])
+@pytest.mark.parametrize("q", [0.5, 1e-2, 1e-4])
+def test_krylov_chunks_stop_at_the_goal(emul, cg, q):
+    """A residual that falls by q per iteration to the goal in k iterations: after
+    a first chunk of two no iteration is queued past the one that meets the
+    goal, the k-th in BiCGStab and, in CG, which looks at the residual on entry
+    to an iteration, the (k + 1)-th; k up to eight more than the two, the most
+    that are queued at once."""
+    f = emul.emul_next_chunk
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.c_double] * 3 + [ctypes.c_int] * 4
+    for k in range(3, 10):
+        tol2 = q ** (k - 0.5)
+        rr_last, it_last, it = 1.0, 0, 2
+        last = k + cg
+        while it < last:
+            rr = q ** (it - cg)
+            n = f(rr_last, rr, tol2, it_last, it, cg, 8)
+            assert n <= last - it, (k, it, n)
+            rr_last, it_last, it = rr, it, it + n
+        assert it == last
+    assert f(1.0, 0.5, 1e-300, 0, 2, cg, 8) == 8  # far from the goal
+    assert f(1.0, 2.0, 1e-3, 0, 2, cg, 8) == 8  # no decrease, no rate
