@@ -699,36 +699,40 @@ __device__ __forceinline__ double cicsamUq(double g, double co) {
   return g >= 0 && g <= 1 ? smin((8. * co * g + (1. - co) * (6. * g + 3.)) / 8., cicsamHc(g, co)) : g;
 }
 
-// Courant number of each cell's outflow over all of its faces, summed in link
-// order (the donor's number in Cicsam.cpp:20-66, once per cell: per face it
-// reads the donor's four faces again)
+// Courant number of a cell's outflow over all of its faces, summed in link order
+// (the donor's number in Cicsam.cpp:20-66)
+__device__ __forceinline__ double courantOf(const MeshDev &M, int c, const double *__restrict__ uF, double dt) {
+  const double v = M.vol[c];
+  double sum = 0.;
+  Dv2 n[4], u[4];
+  auto load = [&](int q, int link) {
+    n[q] = outwardOf(link, M.sf);
+    u[q] = ld2(uF, faceOf(link));
+  };
+  auto add = [&](int q, int) { sum += smax((u[q].x * n[q].x + u[q].y * n[q].y) / v * dt, 0.); };
+  forLinks(M.iptr[c], M.iptr[c + 1], [&](int q, int k) { load(q, M.iface[k]); }, add);
+  for (int k = M.bptr[c]; k < M.bptr[c + 1]; ++k) {
+    load(0, M.bface[k]);
+    add(0, k);
+  }
+  return sum;
+}
 __global__ __launch_bounds__(256) void kCellCourant(MeshDev M, const double *__restrict__ uF, double dt,
                                                     double *__restrict__ co) {
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < M.nCells; c += gridDim.x * blockDim.x) {
-    const double v = M.vol[c];
-    double sum = 0.;
-    Dv2 n[4], u[4];
-    auto load = [&](int q, int link) {
-      n[q] = outwardOf(link, M.sf);
-      u[q] = ld2(uF, faceOf(link));
-    };
-    auto add = [&](int q, int) { sum += smax((u[q].x * n[q].x + u[q].y * n[q].y) / v * dt, 0.); };
-    forLinks(M.iptr[c], M.iptr[c + 1], [&](int q, int k) { load(q, M.iface[k]); }, add);
-    for (int k = M.bptr[c]; k < M.bptr[c + 1]; ++k) {
-      load(0, M.bface[k]);
-      add(0, k);
-    }
-    co[c] = sum;
-  }
+  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < M.nCells; c += gridDim.x * blockDim.x)
+    co[c] = courantOf(M, c, uF, dt);
 }
 
 // cicsam::faceInterpolationWeights, Cicsam.cpp:20-66 (k = 1), one face per
 // thread; boundary faces 0.  cos(2 theta_F) with theta_F = acos(c) is
 // evaluated as 2 c^2 - 1 (c > 1 from rounding stays NaN, as acos makes it).
+// CELLS: the donors' Courant numbers from kCellCourant, once per cell; else
+// formed here, the donor's four faces read again per face.
+template <bool CELLS>
 __global__ __launch_bounds__(256) void kCicsamWeights(MeshDev M, int nFaces, const int *__restrict__ fl,
                                                       const int *__restrict__ fr, const double *__restrict__ uF,
                                                       const double *__restrict__ gC,
-                                                      const double *__restrict__ gradC,
+                                                      const double *__restrict__ gradC, double dt,
                                                       const double *__restrict__ co, double *__restrict__ beta) {
   for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nFaces; f += gridDim.x * blockDim.x) {
     const int l = fl[f], r = fr[f];
@@ -743,7 +747,7 @@ __global__ __launch_bounds__(256) void kCicsamWeights(MeshDev M, int nFaces, con
     const Dv2 cd = ld2(M.cc, d), ca = ld2(M.cc, a);
     const Dv2 rc{ca.x - cd.x, ca.y - cd.y};
     const Dv2 gd = ld2(gradC, d);
-    const double coD = co[d];
+    const double coD = CELLS ? co[d] : courantOf(M, d, uF, dt);
     const double gD = sclamp(gC[d], 0., 1.), gA = sclamp(gC[a], 0., 1.);
     const double gU = sclamp(gA - 2. * (rc.x * gd.x + rc.y * gd.y), 0., 1.);
     double gDT = (gD - gU) / (gA - gU);
@@ -1596,10 +1600,13 @@ int phase_hip_cicsam_weights(phase_hip_mesh *m, const double *uFace, const doubl
   return guardedM(m, [&] {
     if (!uFace || !gammaCell || !gradGammaCell || !beta) fail(PHASE_HIP_EINVAL, "null field");
     PH_CHECK(hipSetDevice(m->device));
-    hipLaunchKernelGGL(kCellCourant, dim3(g256(m->nCells)), dim3(256), 0, m->stream, meshDev(m), uFace, timeStep,
-                       m->dCourant.p);
-    hipLaunchKernelGGL(kCicsamWeights, dim3(g256(m->nFaces)), dim3(256), 0, m->stream, meshDev(m), m->nFaces,
-                       m->dFL.p, m->dFR.p, uFace, gammaCell, gradGammaCell, m->dCourant.p, beta);
+    const bool cells = courantPerCell(m->nCells, m->maxDeg);
+    if (cells)
+      hipLaunchKernelGGL(kCellCourant, dim3(g256(m->nCells)), dim3(256), 0, m->stream, meshDev(m), uFace, timeStep,
+                         m->dCourant.p);
+    hipLaunchKernelGGL(cells ? kCicsamWeights<true> : kCicsamWeights<false>, dim3(g256(m->nFaces)), dim3(256), 0,
+                       m->stream, meshDev(m), m->nFaces, m->dFL.p, m->dFR.p, uFace, gammaCell, gradGammaCell, timeStep,
+                       m->dCourant.p, beta);
     PH_CHECK(hipGetLastError());
   });
 }

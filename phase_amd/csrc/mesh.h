@@ -27,7 +27,7 @@ struct phase_hip_mesh {
   phase::DBuf<double> dIDot, dIMs, dBDot, dBMs;  // per link: dot(r, Sf_out), |r|^2
   phase::DBuf<int> dIfaceS, dBfaceS;  // per link: the face, kFlip set where Sf points into the cell
   phase::DBuf<double> dFaceD, dFaceW;  // per face: r (interleaved), and the left cell's distance weight
-  phase::DBuf<double> dCourant;        // per cell: work space of the CICSAM weights
+  phase::DBuf<double> dCourant;  // per cell: work space of the CICSAM weights (courantPerCell)
 };
 
 namespace phase {
@@ -39,6 +39,15 @@ struct Dv2 {
 // A vector of the interleaved fields as one 16-byte access (fields of callers
 // are only known to be 8-byte aligned, which the hardware takes).
 typedef double dv2_t __attribute__((ext_vector_type(2), aligned(8)));
+
+// The CICSAM weights form a donor's Courant number per face, its faces read again
+// for each, or first once per cell, a launch of its own: worth it on large meshes
+// of triangles only (per face / per cell: 2,000 triangles 4.3 / 6.1 us, 130,000
+// 11.3 / 13.2, 200,000 17.4 / 17.3, 400,000 31.8 / 28.0, one million 76.2 / 63.3;
+// 16,384 quads 4.3 / 8.6, 500,000 30.5 / 33.2, one million 43.2 / 56.0, two million
+// 103.8 / 104.9).
+constexpr int kCourantCells = 1 << 18;
+inline bool courantPerCell(int nCells, int maxDeg) { return maxDeg <= 3 && nCells > kCourantCells; }
 
 // Link entries of dIfaceS / dBfaceS: the outward test of Face::outwardNorm is a
 // property of the mesh, so the operators read its result with the face instead

@@ -425,7 +425,7 @@ int phase_hip_mesh_create(phase_hip_mesh **out, int device, int nNodes, const do
     m->dBfaceS.alloc(std::max<size_t>(1, m->bface.size()));
     m->dFaceD.alloc(2 * (size_t)m->nFaces);
     m->dFaceW.alloc(m->nFaces);
-    m->dCourant.alloc(nCells);
+    if (courantPerCell(nCells, m->maxDeg)) m->dCourant.alloc(nCells);
     hipLaunchKernelGGL(kCellGeom, dim3(grid1(nCells)), dim3(256), 0, st, nCells, m->dCptr.p, m->dCind.p, m->dXY.p,
                        m->dVol.p, m->dCC.p);
     hipLaunchKernelGGL(kFaceGeom, dim3(grid1(m->nFaces)), dim3(256), 0, st, m->nFaces, m->dFNode1.p, m->dFNode2.p,

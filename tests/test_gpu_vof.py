@@ -69,6 +69,28 @@ def test_weights_flux_properties_bitwise(oracle, hip, case):
         assert same(a.get(), b)
 
 
+@pytest.mark.parametrize("nx", [512, 513])
+def test_weights_large_triangle_meshes_bitwise(oracle, hip, nx):
+    """Above 2^18 triangles the donors' Courant numbers are formed per cell, up to
+    there per face (262,144 and 262,656 of them, quads cut in two)."""
+    xy, cptr, cind = H.rect_case(nx, 256)
+    q = cind.reshape(-1, 4)
+    cind = np.ascontiguousarray(np.c_[q[:, [0, 1, 2]], q[:, [0, 2, 3]]].reshape(-1), np.int32)
+    cptr = 3 * np.arange(len(cind) // 3 + 1, dtype=np.int32)
+    om, hm = oracle.Mesh(xy, cptr, cind), hip.HipMesh(xy, cptr, cind)
+    N, F = om.n_cells, om.n_faces
+    assert N == 512 * nx
+    rng = np.random.default_rng(nx)
+    u = closed_box_velocity(om.faces()["centroid"])
+    g = rng.random(N)
+    gradc = 100.0 * rng.standard_normal(2 * N)
+    ref = oracle.cicsam_weights(om, u, g, gradc, 1e-3)
+    d_beta = hip.DeviceArray.zeros(F)
+    hm.cicsam_weights(hip.DeviceArray(u), hip.DeviceArray(g), hip.DeviceArray(gradc), 1e-3, d_beta)
+    assert same(d_beta.get(), ref)
+    assert np.any((ref > 0) & (ref < 1))
+
+
 @pytest.mark.parametrize("theta", [0.5, 1.0])
 def test_cicsam_div_bitwise(oracle, hip, case, theta):
     om, hm, u, gamma = case
