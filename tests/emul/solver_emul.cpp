@@ -1,11 +1,13 @@
 // CPU emulation of the device solver's layout and kernels (test-only).
 //
 // Builds the product's ordering (phase_amd/csrc/ordering.cpp) and replays the
-// SELL-64 SpMV, the ILU(0) factorisation and both triangular sweeps exactly as
-// the gfx950 kernels in solver_kernels.h do -- block by block in ticket order,
-// level by level inside a block -- while checking every array index against
-// its bounds and every dependency against the schedule (a predecessor block
-// must already be finished, an in-block dependency must sit at a lower level).
+// SELL-64 SpMV, the ILU(0) factorisation (a block's entries in its LDS array) and
+// both triangular sweeps (in-block levels out of registers and through the LDS
+// array) as the gfx950 kernels in solver_kernels.h do -- block by block in launch
+// order, level by level inside a block -- while checking every array index,
+// those into LDS included, against its bounds and every dependency against the
+// schedule (a predecessor block must already be finished, an in-block dependency
+// must sit at a lower level).
 // The results are compared with the oracle by tests/test_ordering_emul.py.
 #include <algorithm>
 #include <cmath>
@@ -73,11 +75,8 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
     }
     const size_t nFac = (size_t)o.nLSlots + o.nUSlots + n;
     REQ(o.facSrc.size() == nFac, "facSrc size");
-    std::vector<double> fac(nFac);
-    for (size_t i = 0; i < nFac; ++i) {
-      REQ(o.facSrc[i] < nslots, "facSrc out of range");
-      fac[i] = o.facSrc[i] >= 0 ? vals[o.facSrc[i]] : 0.;
-    }
+    for (size_t i = 0; i < nFac; ++i) REQ(o.facSrc[i] < nslots, "facSrc out of range");
+    std::vector<double> fac(nFac, NAN);  // written by the factorisation only
     // --- SpMV (kSpmv)
     REQ((int)o.sliceOff.size() == o.nSlices + 1, "sliceOff size");
     for (int k = 0; k < n; ++k) {
@@ -137,7 +136,12 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
       }
     }
     std::vector<char> doneBlk(nb, 0), rowDone(n, 0);
-    // --- factorisation (kIluFactor), blocks in ticket order
+    // --- factorisation (kIluFactor), blocks in launch order: a block's entries in
+    // its LDS array, the pivots and first update sources of earlier blocks loaded
+    // before the levels, the results and the inverse diagonal stored at the end
+    int facSlots = 1;
+    for (const BlockInfo &B : o.blocks) facSlots = std::max(facSlots, B.kL + B.kU + 1);
+    REQ((size_t)facSlots * 64 * sizeof(double) <= 65536, "factor block beyond the LDS of a launch");
     for (int b = 0; b < nb; ++b) {
       const BlockInfo &B = o.blocks[b];
       REQ(B.nRows >= 1 && B.nRows <= 64, "block size");
@@ -145,6 +149,58 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
       for (int q = B.predBeg; q < B.predEnd; ++q) {
         REQ(o.pred[q] < b, "pred block not earlier");
         REQ(doneBlk[o.pred[q]], "pred block not finished");
+      }
+      std::vector<double> lds((size_t)facSlots * 64, NAN);
+      auto f = [&](int at) -> double & {
+        REQ(at >= 0 && (size_t)at < lds.size(), "LDS index");
+        return lds[at];
+      };
+      const int uFirst = o.nLSlots + B.uOff, nSlot = B.kL + B.kU;
+      auto place = [&](int s) {
+        if (s < o.nLSlots) return s - B.lOff;
+        if (s < dbase) return s >= uFirst && s < uFirst + (B.kU << 6) ? (B.kL << 6) + s - uFirst : -1;
+        return s - dbase >= B.rowStart && s - dbase < B.rowStart + B.nRows
+                   ? ((B.kL + B.kU) << 6) + s - dbase - B.rowStart
+                   : -1;
+      };
+      // a value of an earlier block, read from memory
+      auto earlier = [&](int s) {
+        REQ(s >= o.nLSlots && (size_t)s < nFac, "off-block factor index");
+        if (s >= dbase) REQ(s - dbase < B.rowStart && rowDone[s - dbase], "off-block pivot not final");
+        else REQ(s < uFirst, "off-block update source not in an earlier block");
+        return fac[s];
+      };
+      // a value of this block: its row must sit at a lower level
+      auto inBlock = [&](int at, int lev) {
+        REQ((at & 63) < B.nRows && o.rows[B.rowStart + (at & 63)].lev < lev, "in-block value not at a lower level");
+        return f(at);
+      };
+      for (int lane = 0; lane < 64; ++lane) {
+        const bool act = lane < B.nRows;
+        for (int e = 0; e <= nSlot; ++e) {
+          int src = -1;
+          if (e < B.kL) src = o.facSrc[lslot(B, e, lane)];
+          else if (e < nSlot) src = o.facSrc[o.nLSlots + uslot(B, e - B.kL, lane)];
+          else if (act) src = o.facSrc[dbase + B.rowStart + lane];
+          f((e << 6) + lane) = src >= 0 ? vals[src] : 0.;
+        }
+      }
+      constexpr int kFacW = 4;
+      struct Ahead {
+        double pv[kFacW], sv[kFacW][2];
+      };
+      std::vector<Ahead> ahead(64);
+      for (int lane = 0; lane < B.nRows; ++lane) {
+        const int nL = o.rows[B.rowStart + lane].nL;
+        for (int e = 0; e < kFacW && e < nL; ++e) {
+          const int s = lslot(B, e, lane), p = dbase + o.lCol[s];
+          ahead[lane].pv[e] = place(p) < 0 ? earlier(p) : NAN;
+          for (int u = 0; u < 2; ++u) {
+            ahead[lane].sv[e][u] = NAN;
+            if (o.updPtr[s] + u < o.updPtr[s + 1] && place(o.updSrc[o.updPtr[s] + u]) < 0)
+              ahead[lane].sv[e][u] = earlier(o.updSrc[o.updPtr[s] + u]);
+          }
+        }
       }
       for (int lev = 0; lev < B.nLev; ++lev) {
         for (int lane = 0; lane < B.nRows; ++lane) {
@@ -156,19 +212,29 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
             const int k = o.lCol[s];
             REQ(k >= 0 && k < row, "L column not below diagonal");
             if (e < ri.nLoff) REQ(k < B.rowStart, "off-block L entry inside block");
-            else REQ(k >= B.rowStart && o.rows[k].lev < lev, "in-block L dependency not at a lower level");
-            REQ(rowDone[k], "L dependency row not finished");
-            const double lik = fac[s] / fac[dbase + k];
-            fac[s] = lik;
+            else REQ(k >= B.rowStart, "in-block L entry outside block");
+            const int pAt = place(dbase + k);
+            const double piv = pAt >= 0 ? inBlock(pAt, lev) : e < kFacW ? ahead[lane].pv[e] : earlier(dbase + k);
+            const double lik = f((e << 6) + lane) / piv;
+            f((e << 6) + lane) = lik;
             REQ(o.updPtr[s] <= o.updPtr[s + 1], "updPtr");
             for (int u = o.updPtr[s]; u < o.updPtr[s + 1]; ++u) {
-              const int dst = o.updDst[u], src = o.updSrc[u];
-              REQ(dst >= 0 && (size_t)dst < nFac && src >= o.nLSlots && src < dbase, "update index");
-              fac[dst] = std::fma(-lik, fac[src], fac[dst]);
+              const int n0 = u - o.updPtr[s], from = place(o.updSrc[u]), to = place(o.updDst[u]);
+              REQ(o.updSrc[u] >= o.nLSlots && o.updSrc[u] < dbase, "update source not a U entry");
+              REQ((to & 63) == lane, "update of another row");
+              const double src = from >= 0               ? inBlock(from, lev)
+                                 : e < kFacW && n0 < 2 ? ahead[lane].sv[e][n0]
+                                                         : earlier(o.updSrc[u]);
+              f(to) = std::fma(-lik, src, f(to));
             }
           }
           rowDone[row] = 1;
         }
+      }
+      for (int lane = 0; lane < 64; ++lane) {
+        for (int e = 0; e < B.kL; ++e) fac[lslot(B, e, lane)] = f((e << 6) + lane);
+        for (int e = 0; e < B.kU; ++e) fac[o.nLSlots + uslot(B, e, lane)] = f(((B.kL + e) << 6) + lane);
+        if (lane < B.nRows) fac[dbase + B.rowStart + lane] = f((nSlot << 6) + lane);
       }
       for (int lane = 0; lane < B.nRows; ++lane) REQ(rowDone[B.rowStart + lane], "row left unprocessed");
       doneBlk[b] = 1;
@@ -210,22 +276,45 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
           acc[lane] = std::fma(-fac[s], y[o.lCol[s]], acc[lane]);
         }
       }
-      for (int lev = 0; lev < B.nLev; ++lev) {
-        for (int lane = 0; lane < B.nRows; ++lane) {
-          const int row = B.rowStart + lane;
-          const RowInfo &ri = o.rows[row];
-          if (ri.lev != lev) continue;
-          for (int e = ri.nLoff; e < ri.nL; ++e) {
-            const int s = lslot(B, e, lane);
-            const int li = o.lCol[s] - B.rowStart;
-            REQ(li >= 0 && li < lane && rowDone[o.lCol[s]], "fwd in-block value not ready");
-            acc[lane] = std::fma(-fac[s], lds[li], acc[lane]);
+      // in-block levels: out of registers, every lane forming its row again at each
+      // level from the others' values of the level before (__shfl), or through the
+      // LDS array where a row is wider than the registers
+      int most = 0;
+      for (int lane = 0; lane < B.nRows; ++lane)
+        most = std::max(most, o.rows[B.rowStart + lane].nL - o.rows[B.rowStart + lane].nLoff);
+      auto entry = [&](int lane, int e, double v, auto &&value) {
+        const int s = lslot(B, e, lane), li = o.lCol[s] - B.rowStart;
+        REQ(li >= 0 && li < lane, "fwd in-block column");
+        return std::fma(-fac[s], value(li), v);
+      };
+      if (most > o.regWidth) {
+        for (int lev = 0; lev < B.nLev; ++lev)
+          for (int lane = 0; lane < B.nRows; ++lane) {
+            const RowInfo &ri = o.rows[B.rowStart + lane];
+            if (ri.lev != lev) continue;
+            for (int e = ri.nLoff; e < ri.nL; ++e)
+              acc[lane] = entry(lane, e, acc[lane], [&](int li) {
+                REQ(o.rows[B.rowStart + li].lev < lev, "fwd in-block value not ready");
+                return lds[li];
+              });
+            lds[lane] = acc[lane];
           }
-          lds[lane] = acc[lane];
-          y[row] = acc[lane];
+      } else {
+        lds = acc;  // rows of level 0 are final
+        for (int lev = 1; lev < B.nLev; ++lev) {
+          const std::vector<double> before = lds;
+          for (int lane = 0; lane < B.nRows; ++lane) {
+            const RowInfo &ri = o.rows[B.rowStart + lane];
+            double v = acc[lane];
+            for (int e = ri.nLoff; e < ri.nL; ++e) v = entry(lane, e, v, [&](int li) { return before[li]; });
+            REQ(ri.lev >= lev || v == lds[lane], "fwd row changed after its level");
+            lds[lane] = v;
+          }
         }
-        for (int lane = 0; lane < B.nRows; ++lane)
-          if (o.rows[B.rowStart + lane].lev == lev) rowDone[B.rowStart + lane] = 1;
+      }
+      for (int lane = 0; lane < B.nRows; ++lane) {
+        y[B.rowStart + lane] = lds[lane];
+        rowDone[B.rowStart + lane] = 1;
       }
       doneBlk[b] = 1;
     }
@@ -252,23 +341,40 @@ extern "C" int emul_run(int n, const int *rowPtr, const int *colInd, const doubl
           soff[lane] = std::fma(fac[o.nLSlots + s], x[o.uCol[s]], soff[lane]);
         }
       }
-      for (int lev = 0; lev < B.nULev; ++lev) {
-        for (int lane = 0; lane < B.nRows; ++lane) {
-          const int row = B.rowStart + lane;
-          const RowInfo &ri = o.rows[row];
-          if (ri.ulev != lev) continue;
-          for (int e = 0; e < ri.nUin; ++e) {
-            const int s = uslot(B, e, lane);
-            const int li = o.uCol[s] - B.rowStart;
-            REQ(li > lane && li < B.nRows && rowDone[o.uCol[s]], "bwd in-block value not ready");
-            acc[lane] = std::fma(-fac[o.nLSlots + s], lds[li], acc[lane]);
-          }
-          acc[lane] = (acc[lane] - soff[lane]) * (1.0 / fac[dbase + row]);
-          lds[lane] = acc[lane];
-          x[row] = acc[lane];
+      int most = 0;
+      for (int lane = 0; lane < B.nRows; ++lane) most = std::max(most, (int)o.rows[B.rowStart + lane].nUin);
+      auto solve = [&](int lane, double v, auto &&value) {
+        const int row = B.rowStart + lane;
+        for (int e = 0; e < o.rows[row].nUin; ++e) {
+          const int s = uslot(B, e, lane), li = o.uCol[s] - B.rowStart;
+          REQ(li > lane && li < B.nRows, "bwd in-block column");
+          v = std::fma(-fac[o.nLSlots + s], value(li), v);
         }
+        return (v - soff[lane]) * (1.0 / fac[dbase + row]);
+      };
+      // through the LDS array: wide rows, and FP64 launches that fill the chip
+      for (int lev = 0; lev < B.nULev; ++lev)
+        for (int lane = 0; lane < B.nRows; ++lane) {
+          if (o.rows[B.rowStart + lane].ulev != lev) continue;
+          lds[lane] = solve(lane, acc[lane], [&](int li) {
+            REQ(o.rows[B.rowStart + li].ulev < lev, "bwd in-block value not ready");
+            return lds[li];
+          });
+        }
+      if (most <= o.regWidth) {  // out of registers: the same bits
+        std::vector<double> reg(64, 0.);
         for (int lane = 0; lane < B.nRows; ++lane)
-          if (o.rows[B.rowStart + lane].ulev == lev) rowDone[B.rowStart + lane] = 1;
+          reg[lane] = (acc[lane] - soff[lane]) * (1.0 / fac[dbase + B.rowStart + lane]);
+        for (int lev = 1; lev < B.nULev; ++lev) {
+          const std::vector<double> before = reg;
+          for (int lane = 0; lane < B.nRows; ++lane)
+            reg[lane] = solve(lane, acc[lane], [&](int li) { return before[li]; });
+        }
+        for (int lane = 0; lane < B.nRows; ++lane) REQ(reg[lane] == lds[lane], "bwd forms differ");
+      }
+      for (int lane = 0; lane < B.nRows; ++lane) {
+        x[B.rowStart + lane] = lds[lane];
+        rowDone[B.rowStart + lane] = 1;
       }
       doneBlk[b] = 1;
     }
