@@ -95,7 +95,12 @@ def test_layer_tiles_match_fp64_oracle(hip, oracle, nx, ny):
     rows) and where a workgroup takes two tiles, in the backward kernel only
     (63,001 rows) and in both (90,300 rows: the last workgroups' runs are
     short).  The bounds are those of the test above: BF16 products of unit
-    round-off 2^-9 through six layers and back."""
+    round-off 2^-9 through six layers and back.  Every tile's output is held to
+    three times the whole's (one left out would be wrong by its own size).  A target that lives on one tile, the last or the second (a
+    workgroup's second at the larger sizes), makes the gradient that tile's: left
+    out, it would be wrong by about its own size.  Half of that is the bound
+    there, as the round-off of so few rows does not average out (0.15 over the 25
+    rows of the last tile of 63,001)."""
     from phase_amd import meshgen as G
 
     m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, ny), sigma=0.5)
@@ -121,6 +126,22 @@ def test_layer_tiles_match_fp64_oracle(hip, oracle, nx, ny):
     assert rel(grad, flatten(g_ref)) < 0.12
     again = s.learned_eval(r, z, target)
     assert np.array_equal(out, again[0]) and loss == again[1] and np.array_equal(grad, again[2])
+    n = len(b)
+    perm = s.ilu_export()[0]
+    rms = np.linalg.norm(out_ref) / np.sqrt(n)
+    tiles = np.arange(0, n, 64)
+    size = np.diff(np.append(tiles, n))
+    norm = lambda v: np.sqrt(np.add.reduceat(v[perm] ** 2, tiles))  # noqa: E731
+    assert np.all(norm(out - out_ref) <= 0.1 * np.maximum(norm(out_ref), rms * np.sqrt(size)))
+    assert np.all(norm(out_ref) > 0.15 * rms * np.sqrt(size))  # none so small that a tile of zeros would pass
+    for t in {len(tiles) - 1, 1} if len(tiles) > 1 else ():
+        rows = perm[tiles[t]:tiles[t] + size[t]]
+        # along the output, so that their product, the gradient's scale, does not cancel
+        one = np.zeros(n)
+        one[rows] = out_ref[rows] * (1.0 + 0.3 * rng.standard_normal(len(rows)))
+        loss_ref, g_ref, _ = NO.loss_and_grad(Ah, X, p, one)
+        _, loss, grad = s.learned_eval(r, z, one)
+        assert rel(grad, flatten(g_ref)) < 0.5
 
 
 def test_training_and_learned_mode(hip, system):

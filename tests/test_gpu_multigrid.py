@@ -240,6 +240,28 @@ def test_last_levels_match_direct(hip, oracle, nx, rows, coarse, cycle):
         assert np.array_equal(s.x(), x)
 
 
+@pytest.mark.parametrize("nx,ny", [(512, 512), (513, 512)])
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+def test_prolongation_forms_match_known(hip, oracle, nx, ny, mode):
+    """Up to 2^18 rows the finest level's prolongation runs with the post-smoothing
+    residual, above apart from it.  A solve for a known field reaches its goal in
+    the usual number of iterations and is within cond(A) 1e-10 of the field,
+    cond(A) below 16 nx^2 as in the tests below."""
+    m, (rp, ci, v), b, g, bc = H.pressure_system(oracle, *G.rectilinear(nx, ny), sigma=0.5)
+    x_ref = np.random.default_rng(nx).standard_normal(nx * ny)
+    s = hip.HipSparseMatrixSolver(0, tolerance=1e-10, maxIters=2000, solver="cg", mode=mode,
+                                  preconditioner="multigrid")
+    s.set(rp, ci, v)
+    s.set_rhs(oracle.spmv(rp, ci, v, x_ref))
+    s.solve()
+    x = s.x()
+    assert np.linalg.norm(x - x_ref) <= 16 * nx * nx * 1e-10 * np.linalg.norm(x_ref)
+    assert s.n_iters() <= 60, s.n_iters()
+    s.zero_guess()
+    s.solve()
+    assert np.array_equal(s.x(), x)
+
+
 @pytest.mark.parametrize("mode,most", [("fp64", 208), ("mixed", 242)])
 def test_multigrid_memory(hip, mode, most):
     """Device memory a first multigrid solve of 2^19 rows takes: Krylov and cycle
