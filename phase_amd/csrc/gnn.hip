@@ -470,8 +470,9 @@ __device__ __forceinline__ int tileAt(int f, int chunk) { return f * kTPitch + (
 //   partials of dWsm = [h | agg]^T dpre and db = column sums of dpre
 // The combination with the layer above (dhIn, daggIn, gterm) is formed as it is
 // read, and dpre stays in registers and LDS, so per row the kernel moves
-// 7 x 128 B to and from HBM (dh, pre, h, agg in; dh, dagg in FP32 out) and the
-// neighbours' dagg rows out of L2.  MFMA operands: the data product takes the
+// 11 x 128 B to and from HBM: pre, h and agg in BF16, dh in and out and dagg in and
+// out in FP32 (two each); the neighbours' dagg rows beyond the first reading come
+// out of L2.  MFMA operands: the data product takes the
 // weights first and dpre second, the output features dealt to the weight rows
 // as in the forward layer: a lane holds the same 16 features of its row in dh,
 // dpre and the products.  The

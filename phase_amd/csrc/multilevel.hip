@@ -911,20 +911,24 @@ __global__ __launch_bounds__(kRedBlock) void kMlJacDirection(int n, int nSlices,
 // own every step of it costs a launch's latency (3 to 6 us) for well under a
 // microsecond of work.  Here a step costs a barrier: the rows' matrix entries
 // are read once, into registers (up to tailWidth a row, the rest from L2 at
-// every product), and the vector a product gathers from is in LDS.  Bound by
+// every product; of two and three rows a thread some are kept in scratch memory,
+// 16 to 56 B a lane), and the vector a product gathers from is in LDS.  Bound by
 // what one CU reads from L2: the matrix once and the dense inverse once per
-// cycle.  kMlTail keeps the arithmetic of the launches (each row's products in
-// slot order, the vectors rounded to T, sums in FP64) except for the order of
-// the restriction's and the dots' sums.
-// One K-cycle solve: 25.4 us for 2,500 rows (FP32 vectors, dense 175), 14.9 us for
-// 548 (FP64, dense 115), 12.0 us for 540 (FP32, dense 39); as nine launches 45, 45
-// and 36 us.  The V cycle over 276 rows 4.5 us (three launches: 13 us).  With
-// ILU(0) smoothing 412 rows take 15.6 us a K cycle (FP32; sixteen launches 64 us)
-// and 540 rows 8.9 us a V cycle (FP64; five launches 21 us).
+// cycle.  The products with the level's matrix and the Jacobi smoothing are the
+// launches' (each row in slot order, the vectors rounded to T, sums in FP64).  The
+// restriction, the dots and the dense product (in column segments) sum in
+// another order, and with ILU(0) the substitutions are products with the blocks'
+// inverses, formed in FP64 and rounded to T: the same preconditioner to
+// round-off, which grows with a block's condition.
+// One K-cycle solve: 25.6 us for 2,500 rows (FP32 vectors, dense 175), 16.8 us for
+// 548 (FP64, dense 115), 11.9 us for 540 (FP32, dense 39); as nine launches 45, 45
+// and 36 us.  The V cycle over 276 rows 4.8 us (three launches: 13 us).  With
+// ILU(0) smoothing 412 rows take 15.5 us a K cycle (FP32; sixteen launches 64 us)
+// and 540 rows 8.6 us a V cycle (FP64; five launches 21 us).
 constexpr int kTailBlock = 1024;
 constexpr int kTailInvBytes = 104 * 1024;  // LDS for block inverses, beside at most 52 KB of vectors
 // Rows per thread and dense rows at most.  A fourth row's matrix entries spill
-// (128 to 236 B a lane; three rows 0 to 64), and past 256 dense rows one CU reads
+// (128 to 236 B a lane; three rows 0 to 56), and past 256 dense rows one CU reads
 // the inverse for longer than the launches it saves; an iteration of a solve with
 // the level as launches / in one workgroup: 2,825 rows over 203 dense ones 143 /
 // 127 us (K cycle, FP64; FP32 134 / 116, V cycles 104 / 106 and 100 / 100), 3,087 over 215

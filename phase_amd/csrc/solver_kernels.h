@@ -643,7 +643,7 @@ __device__ __forceinline__ int colourBlock(int blockBase) { return blockBase + x
 // entries and the sources of their first two updates each.  A level then costs
 // divisions and LDS trips, where in global memory each entry was a chain of
 // round trips.  One million quads (FP64, 4 colours, 32,849 blocks): 199 us for
-// the factorisation, 427 with the entries gathered by a launch of its own, the
+// the factorisation, 434 with the entries gathered by a launch of its own, the
 // updates in global memory and the inverse diagonal in a third launch (97 + 330
 // + 7); 500,000 quads (3 colours) 62 against 153; 16,384 quads 11.8 us a colour, 19.7.
 constexpr int kFacW = 4;
@@ -781,9 +781,10 @@ __global__ __launch_bounds__(64) void kIluFactor(IluDev<T> L, int n, const doubl
 // same arithmetic gives the same bits after it), taking its neighbours' values
 // out of their registers (__shfl).  That is one trip through the LDS crossbar
 // per level where a write and a read of an LDS array are two; rows wider than
-// the registers (coarse multigrid levels) keep the array.  The fused launch over
-// 7,168 rows takes 4.5 us in FP32 (6.4 us with the array), 27,264 rows in FP64
-// 5.7 us (7.4), 415,232 rows in FP32 10.0 us (12.0).
+// the registers (coarse multigrid levels) keep the array, and so do the backward
+// levels of FP64 launches that fill the chip (byLevels, solver_launch.h).  The
+// fused launch over 7,168 rows takes 4.4 us in FP32 (6.4 us with the array), 27,264
+// rows in FP64 5.4 us (7.4), 415,232 rows in FP32 9.5 us (12.0).
 
 // Calls f with the largest v of the wavefront (at most W) as a compile-time
 // constant: the level loops skip the entries no row of the block has, with the
