@@ -67,24 +67,25 @@ def measured_traffic(kernel):
 TRACE_FILE = os.path.join(ROOT, "profiles", "kernels_pcorr_poisson_1M.md")
 # kernel names of a rocprofv3 trace -> entries of time_kernels() that time the same launches
 TRACE_KEYS = {
-    "phase::kLSolve<float, 3, 4>": "lsolve32cg_launch", "phase::kLUSolve<float, 3, 4>": "lusolve32cg_launch",
-    "phase::kLSolve<float, 0, 4>": "lsolve32_launch", "phase::kLUSolve<float, 0, 4>": "lusolve32_launch",
-    "phase::kUSolve<float, 4>": "usolve32_launch",
-    "phase::kLSolve<double, 3, 4>": "lsolve64cg_launch", "phase::kLUSolve<double, 3, 4>": "lusolve64cg_launch",
-    "phase::kLSolve<double, 0, 4>": "lsolve64_launch", "phase::kLUSolve<double, 0, 4>": "lusolve64_launch",
-    "phase::kUSolve<double, 4>": "usolve64_launch", "phase::kSpmv<double>": "spmv64",
+    "phase::kLSolve<float, 3, 4>": "lsolve32cg_launch", "phase::kLUSolve<float, 3, 4, true>": "lusolve32cg_launch",
+    "phase::kLSolve<float, 0, 4>": "lsolve32_launch", "phase::kLUSolve<float, 0, 4, true>": "lusolve32_launch",
+    "phase::kUSolve<float, 4, true>": "usolve32_launch",
+    "phase::kLSolve<double, 3, 4>": "lsolve64cg_launch", "phase::kLUSolve<double, 3, 4, false>": "lusolve64cg_launch",
+    "phase::kLSolve<double, 0, 4>": "lsolve64_launch", "phase::kLUSolve<double, 0, 4, false>": "lusolve64_launch",
+    "phase::kUSolve<double, 4, false>": "usolve64_launch", "phase::kSpmv<double>": "spmv64",
     "phase::kMlResid<float, double>": "mlresid32", "phase::kMlResid<double, double>": "mlresid64",
 }
 
 
 def dominant_from_trace():
-    """Kernel name of the first data row of the first table in the committed
-    kernel-trace summary of the headline method (rows sorted by total time)."""
+    """Kernel name of the first row that the timing block times by itself in the
+    committed kernel-trace summary of the headline method (rows sorted by total
+    time; the one-workgroup kernels are not bound by memory and not timed)."""
     try:
         with open(TRACE_FILE) as f:
             for line in f:
                 cells = [c.strip() for c in line.split("|")]
-                if len(cells) > 2 and cells[1].startswith("`phase::"):
+                if len(cells) > 2 and cells[1].strip("`") in TRACE_KEYS:
                     return cells[1].strip("`")
     except OSError:
         pass
@@ -766,9 +767,9 @@ def main():
     # headline: the fastest method that reached the FP64 goal
     ok = {k: v for k, v in results.items() if v["relres"] <= args.tol}
     head = min(ok, key=lambda k: ok[k]["ms_per_step"]) if ok else list(results)[0]
-    # dominant kernel of the headline solve: the top row (largest share of
-    # kernel time) of the committed kernel trace of the headline method; its
-    # launches are timed live above with HIP events
+    # dominant kernel of the headline solve: the largest in the committed kernel
+    # trace of the headline method whose launches are timed live above with HIP
+    # events
     dom_name = dominant_from_trace()
     key = TRACE_KEYS.get(dom_name)
     if key is None or key not in kernels:
